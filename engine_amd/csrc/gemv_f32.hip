@@ -15,9 +15,8 @@
 //    uses them, then the f32 sum X_g of each of its scale groups. A record is
 //    68 dwords (17 x 16 bytes, odd), so 16 lanes' 128-bit reads hit distinct
 //    banks. One member's slice is 17 KB.
-//  - One member: a lane keeps its record in VGPRs (64 floats) for every row it
-//    reduces. Several members: the records stay in LDS and a pass of the
-//    weight ring reads each 4-element piece once per member for all its rows.
+//  - One or two members: a lane keeps its record in VGPRs (64 floats a member)
+//    for every row it reduces. Three to eight: gemv_f32_many_kernel below.
 //
 // Arithmetic of one lane and one unit, per scale group g (32 elements for
 // Q4_K / Q5_K, 16 for Q6_K; crates/gguf/src/lib.rs:596-661):
@@ -84,202 +83,154 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
     asm("" : "+v"(v));
     return v;
 }
-// As opaque(), but volatile: ordered after the previous volatile statements,
-// so nothing computed from the value is hoisted above them (bounds the
-// registers of the many-member passes).
-__device__ __forceinline__ uint32_t pinned(uint32_t v) {
-    asm volatile("" : "+v"(v));
-    return v;
+// ------------------------------------------------- scales and quants of a unit
+//
+// Q4_K / Q5_K: (d*sc, dmin*m) of the lane's groups 2p (a0, b0) and 2p+1 (a1, b1).
+template <int T>
+__device__ __forceinline__ void group_scales(const uint4 h, int p, float& a0, float& a1, float& b0, float& b1) {
+    const float dd = half_bits_to_float(h.x & 0xffffu);
+    const float dmin = half_bits_to_float(h.x >> 16);
+    // six-bit scales / minima of all 8 groups, four per word (lib.rs:573-587)
+    const uint32_t lo_sc = h.y & 0x3f3f3f3fu;
+    const uint32_t lo_mn = h.z & 0x3f3f3f3fu;
+    const uint32_t hi_sc = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+    const uint32_t hi_mn = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
+    const uint32_t scw = (p < 2) ? lo_sc : hi_sc;
+    const uint32_t mnw = (p < 2) ? lo_mn : hi_mn;
+    const int sh = (p & 1) * 16;
+    // Q4_K quants enter as q * 2^-9 (quant_quads): scales carry the 2^9, exactly
+    constexpr float kQScale = (T == kQ4K) ? 512.0f : 1.0f;
+    a0 = (dd * (float)((scw >> sh) & 0xffu)) * kQScale;
+    a1 = (dd * (float)((scw >> (sh + 8)) & 0xffu)) * kQScale;
+    b0 = dmin * (float)((mnw >> sh) & 0xffu);
+    b1 = dmin * (float)((mnw >> (sh + 8)) & 0xffu);
+}
+
+// Q4_K / Q5_K: quants 4j .. 4j+3 of group A = 2p (low nibbles) and B = 2p+1
+// (high nibbles), with Q5_K's fifth bit, as f32.
+template <int T>
+__device__ __forceinline__ void quant_quads(const RowData<T>& d, int j, int p, float (&fa)[4], float (&fb)[4]) {
+    const uint32_t qw[8] = {d.qa.x, d.qa.y, d.qa.z, d.qa.w, d.qb.x, d.qb.y, d.qb.z, d.qb.w};
+    uint32_t qa = qw[j] & 0x0f0f0f0fu;
+    uint32_t qb = (qw[j] >> 4) & 0x0f0f0f0fu;
+    if constexpr (T == kQ4K) {
+        // Bytes 0..15 read as OCP E4M3 are exactly q * 2^-9: two quants per
+        // convert (the 2^9 is folded into the scales).
+        const auto a01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qa, false);
+        const auto a23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qa, true);
+        const auto b01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qb, false);
+        const auto b23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qb, true);
+        fa[0] = a01[0];
+        fa[1] = a01[1];
+        fa[2] = a23[0];
+        fa[3] = a23[1];
+        fb[0] = b01[0];
+        fb[1] = b01[1];
+        fb[2] = b23[0];
+        fb[3] = b23[1];
+    } else {
+        const uint32_t hw[8] = {d.ha.x, d.ha.y, d.ha.z, d.ha.w, d.hb.x, d.hb.y, d.hb.z, d.hb.w};
+        qa = opaque(qa | (((hw[j] >> (2 * p)) & 0x01010101u) << 4));
+        qb = opaque(qb | (((hw[j] >> (2 * p + 1)) & 0x01010101u) << 4));
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            fa[t] = byte_f(qa, t);
+            fb[t] = byte_f(qb, t);
+        }
+    }
+}
+
+// Q6_K: the lane's four d*scale factors and its quant words, windows joined.
+__device__ __forceinline__ void q6_fields(const RowData<kQ6K>& d, int p, float (&a)[4], uint32_t (&law)[4],
+                                          uint32_t (&lbw)[4], uint32_t (&qhw)[4]) {
+    const int c = p >> 1, s = p & 1;
+    const uint4 la = funnel(d.la, d.la_t, d.shift);
+    const uint4 lb = funnel(d.lb, d.lb_t, d.shift);
+    const uint4 qh = funnel(d.qh, d.qh_t, d.shift);
+    const uint4 sc = funnel(d.sc, d.sc_t, d.shift);  // int8 scales
+    const float dd = half_bits_to_float(d.d16);
+    const uint32_t w0 = c ? sc.z : sc.x;  // scales 8c+0..8c+3
+    const uint32_t w1 = c ? sc.w : sc.y;  // scales 8c+4..8c+7
+    a[0] = dd * (float)(int8_t)((w0 >> (8 * s)) & 0xffu);
+    a[1] = dd * (float)(int8_t)((w0 >> (8 * (2 + s))) & 0xffu);
+    a[2] = dd * (float)(int8_t)((w1 >> (8 * s)) & 0xffu);
+    a[3] = dd * (float)(int8_t)((w1 >> (8 * (2 + s))) & 0xffu);
+    law[0] = la.x; law[1] = la.y; law[2] = la.z; law[3] = la.w;
+    lbw[0] = lb.x; lbw[1] = lb.y; lbw[2] = lb.z; lbw[3] = lb.w;
+    qhw[0] = qh.x; qhw[1] = qh.y; qhw[2] = qh.z; qhw[3] = qh.w;
+}
+
+// Q6_K: four quants (0..63) of 16-element group v from its low-nibble word
+// (la for even v, lb for odd) and high-bit word; the -32 enters through X_v.
+__device__ __forceinline__ void q6_quad(uint32_t lw, uint32_t qh, int v, float (&f)[4]) {
+    uint32_t q;
+    if (v == 0) q = (lw & 0x0f0f0f0fu) | ((qh << 4) & 0x30303030u);
+    else if (v == 1) q = (lw & 0x0f0f0f0fu) | ((qh << 2) & 0x30303030u);
+    else if (v == 2) q = ((lw >> 4) & 0x0f0f0f0fu) | (qh & 0x30303030u);
+    else q = ((lw >> 4) & 0x0f0f0f0fu) | ((qh >> 2) & 0x30303030u);
+    q = opaque(q);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) f[t] = byte_f(q, t);
 }
 
 // --------------------------------------------------------- lane dot product
 //
-// part[r][m] = this lane's share of row r . x_m for one unit. xf(m, i) returns
-// the i-th float4 of member m's lane record, sf(m, g) its group sum X_g. Each
-// (r, m) pair sees the same operation sequence whatever NR and MT are.
-template <int T, int NR, int MT, class XF, class SF>
-__device__ __forceinline__ void rows_dot(const RowData<T> (&d)[NR], int p, XF xf, SF sf, float (&part)[NR][MT]) {
+// part[m] = this lane's share of the unit's row . x_m. xf(m, i) returns the
+// i-th float4 of member m's lane record, sf(m, g) its group sum X_g. Each
+// member sees the same operation sequence whatever MT is.
+template <int T, int MT, class XF, class SF>
+__device__ __forceinline__ void row_dot(const RowData<T>& d, int p, XF xf, SF sf, float (&part)[MT]) {
+    auto mac4 = [](const float (&f)[4], const float4 x, float s) {
+        s = __builtin_fmaf(f[0], x.x, s);
+        s = __builtin_fmaf(f[1], x.y, s);
+        s = __builtin_fmaf(f[2], x.z, s);
+        return __builtin_fmaf(f[3], x.w, s);
+    };
     if constexpr (T == kQ4K || T == kQ5K) {
-        float a0[NR], a1[NR], b0[NR], b1[NR];
+        float a0, a1, b0, b1;
+        group_scales<T>(d.h, p, a0, a1, b0, b1);
+        float sA[MT], sB[MT];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const uint4 h = d[r].h;
-            const float dd = half_bits_to_float(h.x & 0xffffu);
-            const float dmin = half_bits_to_float(h.x >> 16);
-            // six-bit scales / minima of all 8 groups, four per word (lib.rs:573-587)
-            const uint32_t lo_sc = h.y & 0x3f3f3f3fu;
-            const uint32_t lo_mn = h.z & 0x3f3f3f3fu;
-            const uint32_t hi_sc = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
-            const uint32_t hi_mn = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
-            const uint32_t scw = (p < 2) ? lo_sc : hi_sc;
-            const uint32_t mnw = (p < 2) ? lo_mn : hi_mn;
-            const int sh = (p & 1) * 16;
-            // Q4_K quants enter as q * 2^-9 (see below): scales carry the 2^9, exactly
-            constexpr float kQScale = (T == kQ4K) ? 512.0f : 1.0f;
-            a0[r] = (dd * (float)((scw >> sh) & 0xffu)) * kQScale;
-            a1[r] = (dd * (float)((scw >> (sh + 8)) & 0xffu)) * kQScale;
-            b0[r] = dmin * (float)((mnw >> sh) & 0xffu);
-            b1[r] = dmin * (float)((mnw >> (sh + 8)) & 0xffu);
-        }
-        float sA[NR][MT], sB[NR][MT];
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) sA[r][m] = sB[r][m] = 0.f;
+        for (int m = 0; m < MT; ++m) sA[m] = sB[m] = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            // group A = 2p (low nibbles), group B = 2p+1 (high nibbles), 5th bit for Q5_K
-            float fa[NR][4], fb[NR][4];
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const uint32_t qw[8] = {d[r].qa.x, d[r].qa.y, d[r].qa.z, d[r].qa.w,
-                                        d[r].qb.x, d[r].qb.y, d[r].qb.z, d[r].qb.w};
-                const uint32_t w = (NR * MT > 2) ? pinned(qw[j]) : qw[j];
-                uint32_t qa = w & 0x0f0f0f0fu;
-                uint32_t qb = (w >> 4) & 0x0f0f0f0fu;
-                if constexpr (T == kQ5K) {
-                    const uint32_t hw[8] = {d[r].ha.x, d[r].ha.y, d[r].ha.z, d[r].ha.w,
-                                            d[r].hb.x, d[r].hb.y, d[r].hb.z, d[r].hb.w};
-                    qa |= ((hw[j] >> (2 * p)) & 0x01010101u) << 4;
-                    qb |= ((hw[j] >> (2 * p + 1)) & 0x01010101u) << 4;
-                }
-                if constexpr (T == kQ4K) {
-                    // Bytes 0..15 read as OCP E4M3 are exactly q * 2^-9: two
-                    // quants per convert (the 2^9 is folded into the scales).
-                    const auto a01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qa, false);
-                    const auto a23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qa, true);
-                    const auto b01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qb, false);
-                    const auto b23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qb, true);
-                    fa[r][0] = a01[0];
-                    fa[r][1] = a01[1];
-                    fa[r][2] = a23[0];
-                    fa[r][3] = a23[1];
-                    fb[r][0] = b01[0];
-                    fb[r][1] = b01[1];
-                    fb[r][2] = b23[0];
-                    fb[r][3] = b23[1];
-                } else {
-                    qa = opaque(qa);
-                    qb = opaque(qb);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        fa[r][t] = byte_f(qa, t);
-                        fb[r][t] = byte_f(qb, t);
-                    }
-                }
-            }
+            float fa[4], fb[4];
+            quant_quads<T>(d, j, p, fa, fb);
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const float4 xa = xf(m, j);
-                const float4 xb = xf(m, 8 + j);
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    sA[r][m] = __builtin_fmaf(fa[r][0], xa.x, sA[r][m]);
-                    sA[r][m] = __builtin_fmaf(fa[r][1], xa.y, sA[r][m]);
-                    sA[r][m] = __builtin_fmaf(fa[r][2], xa.z, sA[r][m]);
-                    sA[r][m] = __builtin_fmaf(fa[r][3], xa.w, sA[r][m]);
-                    sB[r][m] = __builtin_fmaf(fb[r][0], xb.x, sB[r][m]);
-                    sB[r][m] = __builtin_fmaf(fb[r][1], xb.y, sB[r][m]);
-                    sB[r][m] = __builtin_fmaf(fb[r][2], xb.z, sB[r][m]);
-                    sB[r][m] = __builtin_fmaf(fb[r][3], xb.w, sB[r][m]);
-                }
-                // Many accumulators: an empty volatile statement on them after
-                // each member keeps the FMAs next to the reads they consume.
-                if constexpr (NR * MT > 2) {
-#pragma unroll
-                    for (int r = 0; r < NR; ++r) asm volatile("" : "+v"(sA[r][m]), "+v"(sB[r][m]));
-                }
+                sA[m] = mac4(fa, xf(m, j), sA[m]);
+                sB[m] = mac4(fb, xf(m, 8 + j), sB[m]);
             }
         }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const float xA = sf(m, 0), xB = sf(m, 1);
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const float tA = __builtin_fmaf(a0[r], sA[r][m], -(b0[r] * xA));
-                const float tB = __builtin_fmaf(a1[r], sB[r][m], -(b1[r] * xB));
-                part[r][m] = tA + tB;
-            }
+            const float tA = __builtin_fmaf(a0, sA[m], -(b0 * sf(m, 0)));
+            const float tB = __builtin_fmaf(a1, sB[m], -(b1 * sf(m, 1)));
+            part[m] = tA + tB;
         }
     } else {
-        const int c = p >> 1, s = p & 1;
-        float a[NR][4];
-        uint32_t law[NR][4], lbw[NR][4], qhw[NR][4];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const uint32_t sh = d[r].shift;
-            const uint4 la = funnel(d[r].la, d[r].la_t, sh);
-            const uint4 lb = funnel(d[r].lb, d[r].lb_t, sh);
-            const uint4 qh = funnel(d[r].qh, d[r].qh_t, sh);
-            const uint4 sc = funnel(d[r].sc, d[r].sc_t, sh);  // int8 scales
-            const float dd = half_bits_to_float(d[r].d16);
-            const uint32_t w0 = c ? sc.z : sc.x;  // scales 8c+0..8c+3
-            const uint32_t w1 = c ? sc.w : sc.y;  // scales 8c+4..8c+7
-            a[r][0] = dd * (float)(int8_t)((w0 >> (8 * s)) & 0xffu);
-            a[r][1] = dd * (float)(int8_t)((w0 >> (8 * (2 + s))) & 0xffu);
-            a[r][2] = dd * (float)(int8_t)((w1 >> (8 * s)) & 0xffu);
-            a[r][3] = dd * (float)(int8_t)((w1 >> (8 * (2 + s))) & 0xffu);
-            law[r][0] = la.x; law[r][1] = la.y; law[r][2] = la.z; law[r][3] = la.w;
-            lbw[r][0] = lb.x; lbw[r][1] = lb.y; lbw[r][2] = lb.z; lbw[r][3] = lb.w;
-            qhw[r][0] = qh.x; qhw[r][1] = qh.y; qhw[r][2] = qh.z; qhw[r][3] = qh.w;
-        }
-        // One 16-element group v at a time: quants 0..63 of group v are
-        // element 16v + 4j + t of the lane's record (the -32 offset enters
-        // through X_v).
-        float acc[NR][MT];
+        float a[4];
+        uint32_t law[4], lbw[4], qhw[4];
+        q6_fields(d, p, a, law, lbw, qhw);
+        // one 16-element group v at a time: element 16v + 4j + t of the lane's record
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            float sv[NR][MT];
+            float sv[MT];
 #pragma unroll
-            for (int r = 0; r < NR; ++r)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) sv[r][m] = 0.f;
+            for (int m = 0; m < MT; ++m) sv[m] = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                float f[NR][4];
+                float f[4];
+                q6_quad((v & 1) ? lbw[j] : law[j], qhw[j], v, f);
 #pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    uint32_t q;
-                    const uint32_t lw = (NR * MT > 2) ? pinned((v & 1) ? lbw[r][j] : law[r][j])
-                                                      : ((v & 1) ? lbw[r][j] : law[r][j]);
-                    if (v == 0) q = (lw & 0x0f0f0f0fu) | ((qhw[r][j] << 4) & 0x30303030u);
-                    else if (v == 1) q = (lw & 0x0f0f0f0fu) | ((qhw[r][j] << 2) & 0x30303030u);
-                    else if (v == 2) q = ((lw >> 4) & 0x0f0f0f0fu) | (qhw[r][j] & 0x30303030u);
-                    else q = ((lw >> 4) & 0x0f0f0f0fu) | ((qhw[r][j] >> 2) & 0x30303030u);
-                    q = opaque(q);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) f[r][t] = byte_f(q, t);
-                }
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    const float4 xv = xf(m, 4 * v + j);
-#pragma unroll
-                    for (int r = 0; r < NR; ++r) {
-                        sv[r][m] = __builtin_fmaf(f[r][0], xv.x, sv[r][m]);
-                        sv[r][m] = __builtin_fmaf(f[r][1], xv.y, sv[r][m]);
-                        sv[r][m] = __builtin_fmaf(f[r][2], xv.z, sv[r][m]);
-                        sv[r][m] = __builtin_fmaf(f[r][3], xv.w, sv[r][m]);
-                    }
-                    if constexpr (NR * MT > 2) {
-#pragma unroll
-                        for (int r = 0; r < NR; ++r) asm volatile("" : "+v"(sv[r][m]));
-                    }
-                }
+                for (int m = 0; m < MT; ++m) sv[m] = mac4(f, xf(m, 4 * v + j), sv[m]);
             }
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const float x32 = 32.0f * sf(m, v);  // exact
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    const float t = a[r][v] * (sv[r][m] - x32);
-                    acc[r][m] = (v == 0) ? t : acc[r][m] + t;
-                }
+                const float t = a[v] * (sv[m] - 32.0f * sf(m, v));  // 32 X exact
+                part[m] = (v == 0) ? t : part[m] + t;
             }
         }
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) part[r][m] = acc[r][m];
     }
 }
 
@@ -296,10 +247,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
     static_assert(NBUF % GROUP == 0, "the ring holds whole row groups");
     static_assert(!SPLIT || (ONE_SLICE && !PAIR && PRO == kProPlain), "slice splits are plain one-slice passes");
     static_assert(!PAIR || (ONE_SLICE && NBUF % 2 == 0), "pairs are whole ring slots of one-slice rows");
-    static_assert(MT <= 2 || ONE_SLICE, "several members stage one slice");
+    static_assert(MT <= 2, "lane records are held in VGPRs");
     constexpr bool NORM = PRO == kProNorm;
     constexpr bool SWIGLU = PRO == kProSwiglu;
-    constexpr bool XREG = MT <= 2;  // lane records held in VGPRs
     constexpr int G = F32Rec<T>::groups;
     constexpr int STRIDE = F32Rec<T>::stride;
     constexpr int BB = BlockTraits<T>::bytes;
@@ -307,7 +257,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
     constexpr int NBW = (NBMAX + WAVES - 1) / WAVES;  // staging blocks per wave
     extern __shared__ float xs[];                     // [MT][slices][64 records][STRIDE]
     __shared__ float ssq_s[NORM ? MT : 1][NORM ? NBMAX : 1];
-    __shared__ __attribute__((aligned(16))) float epi[XREG ? 4 : WAVES * 128];  // many-member pass epilogue, 512 B per wave
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -522,216 +471,507 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
     const __amdgpu_buffer_rsrc_t partial_r =
         make_rsrc(args.partial, SPLIT ? (uint32_t)gridDim.y * (uint32_t)members * (uint32_t)args.total_rows * 4u : 0u);
 
-    if constexpr (!XREG) {
-        // ---- several members, one slice: passes over the whole ring. Each
-        // pass reads every 4-element piece of a member's record once and
-        // applies it to the ring's rows; then the ring is refilled. The last
-        // pass reduces only the wave's remaining NR rows (a wave's share of a
-        // short launch is often fewer rows than the ring holds).
-        const float* rec_base = xs + lane * STRIDE;
-        auto xf = [&](int m, int i) { return *reinterpret_cast<const float4*>(rec_base + m * 64 * STRIDE + 4 * i); };
-        auto sf = [&](int m, int g) { return rec_base[m * 64 * STRIDE + 64 + g]; };
-        int crow = r_begin;
-        float* const ep = epi + wave * 128;  // [4 lane rows][32 values]
-        const int vl = lane & 31;
-        float inv_l = inv[0];  // the RMSNorm factor of this lane's member
+    // ---- one or two members: records in VGPRs; the ring is reduced one
+    // unit at a time and each slot refilled with the unit NBUF ahead.
+    float4 xq[MT][16];
+    float xg[MT][G];
+    auto read_rec = [&](int slice) {
 #pragma unroll
-        for (int m = 1; m < MT; ++m)
-            if (vl % MT == m) inv_l = inv[m];
-        auto pass = [&](auto refill_const, auto nr_const) {
-            constexpr bool REFILL = decltype(refill_const)::value;
-            constexpr int NR = decltype(nr_const)::value;
-            static_assert(NR >= 1 && NR <= NBUF && (REFILL ? NR == NBUF : true), "full passes reduce the whole ring");
-            static_assert(NR * MT <= 32 && MT % 4 == 0, "a pass's values fit lanes 0-31 in whole float4s");
-            // The records never change, but keeping all of them in registers
-            // across passes would spill: re-read them every pass.
-            asm volatile("" ::: "memory");
-            float part[NR][MT];
-            rows_dot<T, NR, MT>(reinterpret_cast<const RowData<T>(&)[NR]>(ring), p, xf, sf, part);
-            if constexpr (REFILL) {
+        for (int m = 0; m < MT; ++m) {
+            const float* src = xs + ((m * slices + slice) * 64 + lane) * STRIDE;
 #pragma unroll
-                for (int r = 0; r < NBUF; ++r) load_next(ring[r], r);
-            }
-            // Epilogue. Each (row r, member m) value's 16-lane row sums (the
-            // DPP steps of wave_sum_uniform) go through this wave's LDS
-            // scratch, and lane v = r * MT + m finishes value v: the row sums
-            // added (r0 + r1) + (r2 + r3), the RMSNorm factor, SwiGLU, the
-            // store. Every value sees wave_sum_uniform's operations in its
-            // order, so the bits equal the single-member launch's, and the
-            // per-value work runs once across lanes instead of once per value.
+            for (int i = 0; i < 16; ++i) xq[m][i] = *reinterpret_cast<const float4*>(src + 4 * i);
+            const float4 sums = *reinterpret_cast<const float4*>(src + 64);
+            const float sv[4] = {sums.x, sums.y, sums.z, sums.w};
 #pragma unroll
-            for (int r = 0; r < NR; ++r)
+            for (int g = 0; g < G; ++g) xg[m][g] = sv[g];
+        }
+    };
+    auto xf = [&](int m, int i) { return xq[m][i]; };
+    auto sf = [&](int m, int g) { return xg[m][g]; };
+    if constexpr (ONE_SLICE) read_rec(0);
+
+    int crow = r_begin, cslice = 0;
+    constexpr int kAcc = ONE_SLICE ? 1 : GROUP;
+    float acc[kAcc][MT];
+    float gk[MT];
 #pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    float v = part[r][m];
-                    v = dpp_step<0xb1>(v);   // quad_perm [1,0,3,2]
-                    v = dpp_step<0x4e>(v);   // quad_perm [2,3,0,1]
-                    v = dpp_step<0x141>(v);  // row_half_mirror
-                    v = dpp_step<0x140>(v);  // row_mirror
-                    part[r][m] = v;
-                }
-            if ((lane & 15) == 0) {
-                float* dst = ep + 32 * (lane >> 4);
+    for (int r = 0; r < kAcc; ++r)
 #pragma unroll
-                for (int i = 0; i < NR * MT; i += 4)
-                    *reinterpret_cast<float4*>(dst + i) =
-                        float4{part[(i + 0) / MT][(i + 0) % MT], part[(i + 1) / MT][(i + 1) % MT],
-                               part[(i + 2) / MT][(i + 2) % MT], part[(i + 3) / MT][(i + 3) % MT]};
-            }
-            // (one wave's LDS operations complete in order: no barrier)
-            auto total_of = [&](int i) { return (ep[i] + ep[32 + i]) + (ep[64 + i] + ep[96 + i]); };
-            const int vr = vl / MT, vm = vl % MT;  // this lane's value: row crow + vr, member vm
-            const int row = crow + vr;
-            // lanes 32-63 repeat lanes 0-31's values and store nothing
-            const bool mine = lane < 32 && vl < NR * MT && row < r_end && vm < members;
+        for (int m = 0; m < MT; ++m) acc[r][m] = 0.f;
+    auto consume = [&](const RowData<T>& d, int r) {
+        if constexpr (!ONE_SLICE) {
+            if (r % GROUP == 0) read_rec(cslice);
+        }
+        float part[MT];
+        row_dot<T, MT>(d, p, xf, sf, part);
+        const int ai = ONE_SLICE ? 0 : r % GROUP;
+        const int row = ONE_SLICE ? crow : crow + r % GROUP;
+        const bool last = ONE_SLICE || cslice == slices - 1;
+        int mat, local, rows_mat;
+        __amdgpu_buffer_rsrc_t yr;
+        if constexpr (kCursor) {
+            if (row < r_end) seek(ccur, row, true);
+            yr = ccur.rs;
+            local = row - ccur.start;
+            rows_mat = ccur.rows_mat;
+        } else if constexpr (PAIR) {
+            yr = pair_y;
+            local = row >> 1;
+            rows_mat = pair_rows;
+        } else {
+            locate(row < r_end ? row : r_begin, mat, local);
+            yr = pick_y(mat, rows_mat);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const float ps = wave_sum_uniform(part[m]);
+            acc[ai][m] = (ONE_SLICE || cslice == 0) ? ps : acc[ai][m] + ps;
+            const float total = acc[ai][m] * inv[m];
+            const uint32_t off = (last && row < r_end && lane == 0 && m < members)
+                                     ? (uint32_t)(m * rows_mat + local) * 4u
+                                     : kOutOfRange;
             if constexpr (SPLIT) {
-                const float ps = total_of(vl);
-                const uint32_t off = mine ? (uint32_t)((slice0 * members + vm) * args.total_rows + row) * 4u : kOutOfRange;
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ps), partial_r, (int)off, 0, 0);
+                // this workgroup's slice total P_s, as the several-member pass stores it
+                const uint32_t poff = (row < r_end && lane == 0 && m < members)
+                                          ? (uint32_t)((slice0 * members + m) * args.total_rows + row) * 4u
+                                          : kOutOfRange;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ps), partial_r, (int)poff, 0, 0);
             } else if constexpr (PAIR) {
-                // gate rows are even, each followed by its up row: lane v
-                // (gate) also adds value v + MT (up)
-                const bool gate = (vr & 1) == 0 && vl + MT < 32;
-                const float g = total_of(vl) * inv_l;
-                const float u = total_of(gate ? vl + MT : vl) * inv_l;
-                const uint32_t off = (mine && gate) ? (uint32_t)(vm * pair_rows + (row >> 1)) * 4u : kOutOfRange;
-                put(swiglu(g, u), pair_y, off);
-            } else {
-                const float total = total_of(vl) * inv_l;
-                // rows move forward; the output resource can change at a
-                // matrix boundary inside the pass, so one store per row
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    const int rr = crow + r;
-                    if (rr < r_end) seek(ccur, rr, true);
-                    const uint32_t off =
-                        (mine && vr == r) ? (uint32_t)(vm * ccur.rows_mat + (rr - ccur.start)) * 4u : kOutOfRange;
-                    put(total, ccur.rs, off);
-                }
-            }
-            crow += NBUF;
-        };
-        const int rows_w = r_end - r_begin;
-        const int passes = (rows_w + NBUF - 1) / NBUF;
-        using Full = std::integral_constant<int, NBUF>;
-        for (int ps = 0; ps + 1 < passes; ++ps) pass(std::true_type{}, Full{});
-        if (passes == 0) return;
-        // 1..NBUF rows left (wave-uniform); gate/up pairs leave an even count
-        const int left = rows_w - (passes - 1) * NBUF;
-        if constexpr (!PAIR) {
-            if (left == 1) return pass(std::false_type{}, std::integral_constant<int, 1>{});
-        }
-        if constexpr (NBUF > 2) {
-            if (left == 2) return pass(std::false_type{}, std::integral_constant<int, 2>{});
-        }
-        if constexpr (NBUF > 3 && !PAIR) {
-            if (left == 3) return pass(std::false_type{}, std::integral_constant<int, 3>{});
-        }
-        pass(std::false_type{}, Full{});
-        return;
-    } else {
-        // ---- one or two members: records in VGPRs; the ring is reduced one
-        // unit at a time and each slot refilled with the unit NBUF ahead.
-        float4 xq[MT][16];
-        float xg[MT][G];
-        auto read_rec = [&](int slice) {
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                const float* src = xs + ((m * slices + slice) * 64 + lane) * STRIDE;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) xq[m][i] = *reinterpret_cast<const float4*>(src + 4 * i);
-                const float4 sums = *reinterpret_cast<const float4*>(src + 64);
-                const float sv[4] = {sums.x, sums.y, sums.z, sums.w};
-#pragma unroll
-                for (int g = 0; g < G; ++g) xg[m][g] = sv[g];
-            }
-        };
-        auto xf = [&](int m, int i) { return xq[m][i]; };
-        auto sf = [&](int m, int g) { return xg[m][g]; };
-        if constexpr (ONE_SLICE) read_rec(0);
-
-        int crow = r_begin, cslice = 0;
-        constexpr int kAcc = ONE_SLICE ? 1 : GROUP;
-        float acc[kAcc][MT];
-        float gk[MT];
-#pragma unroll
-        for (int r = 0; r < kAcc; ++r)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) acc[r][m] = 0.f;
-        auto consume = [&](const RowData<T>& d, int r) {
-            if constexpr (!ONE_SLICE) {
-                if (r % GROUP == 0) read_rec(cslice);
-            }
-            const RowData<T> one[1] = {d};
-            float part[1][MT];
-            rows_dot<T, 1, MT>(one, p, xf, sf, part);
-            const int ai = ONE_SLICE ? 0 : r % GROUP;
-            const int row = ONE_SLICE ? crow : crow + r % GROUP;
-            const bool last = ONE_SLICE || cslice == slices - 1;
-            int mat, local, rows_mat;
-            __amdgpu_buffer_rsrc_t yr;
-            if constexpr (kCursor) {
-                if (row < r_end) seek(ccur, row, true);
-                yr = ccur.rs;
-                local = row - ccur.start;
-                rows_mat = ccur.rows_mat;
-            } else if constexpr (PAIR) {
-                yr = pair_y;
-                local = row >> 1;
-                rows_mat = pair_rows;
-            } else {
-                locate(row < r_end ? row : r_begin, mat, local);
-                yr = pick_y(mat, rows_mat);
-            }
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                const float ps = wave_sum_uniform(part[0][m]);
-                acc[ai][m] = (ONE_SLICE || cslice == 0) ? ps : acc[ai][m] + ps;
-                const float total = acc[ai][m] * inv[m];
-                const uint32_t off = (last && row < r_end && lane == 0 && m < members)
-                                         ? (uint32_t)(m * rows_mat + local) * 4u
-                                         : kOutOfRange;
-                if constexpr (SPLIT) {
-                    // this workgroup's slice total P_s, as the several-member pass stores it
-                    const uint32_t poff = (row < r_end && lane == 0 && m < members)
-                                              ? (uint32_t)((slice0 * members + m) * args.total_rows + row) * 4u
-                                              : kOutOfRange;
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ps), partial_r, (int)poff, 0, 0);
-                } else if constexpr (PAIR) {
-                    if (r % 2 == 0) {
-                        gk[m] = total;
-                    } else {
-                        put(swiglu(gk[m], total), yr, off);
-                    }
+                if (r % 2 == 0) {
+                    gk[m] = total;
                 } else {
-                    put(total, yr, off);
+                    put(swiglu(gk[m], total), yr, off);
+                }
+            } else {
+                put(total, yr, off);
+            }
+        }
+        if constexpr (ONE_SLICE) {
+            ++crow;
+        } else if (r % GROUP == GROUP - 1 && ++cslice == slices) {
+            cslice = 0;
+            crow += GROUP;
+        }
+    };
+
+    const int rows_w = r_end - r_begin;
+    const int units = ONE_SLICE ? rows_w : (rows_w + GROUP - 1) / GROUP * GROUP * slices;
+    const int passes = (units + NBUF - 1) / NBUF;
+    for (int ps = 0; ps + 1 < passes; ++ps) {
+#pragma unroll
+        for (int r = 0; r < NBUF; ++r) {
+            consume(ring[r], r);
+            load_next(ring[r], r);
+        }
+    }
+    if (passes > 0) {
+        const int left = units - (passes - 1) * NBUF;
+#pragma unroll
+        for (int r = 0; r < NBUF; ++r) {
+            if (r < left) consume(ring[r], r);
+        }
+    }
+}
+
+namespace {
+
+// ------------------------------------------- three to eight members, MFMA
+//
+// gemv_f32_many_kernel: the same rows for 3..8 members, one slice per
+// workgroup. The products run on v_mfma_f32_4x4x1_16b_f32: 16 independent
+// 4 x 4 outer products, D[i][j] += x_i * q_j, each element one fused f32
+// multiply-add (checked bit for bit against fmaf over normal, denormal,
+// overflowing, infinite and NaN operands), so a chain of them over a scale
+// group's elements is the S_g of the single-member kernel, in its order.
+//
+// Mapping. A wave owns one quarter of the slice (4 super-blocks, 16 lane
+// records) and walks units of 4 rows x that quarter: lane l holds record
+// l >> 2 of row l & 3 as the B operand, and in VGPRs, for the whole launch,
+// the activations of member (l & 3) (and 4 + (l & 3)) at that record as the A
+// operand. The accumulator of lane l then holds its own row and record for
+// members 0..3, so scales and minima apply where they were loaded, and the
+// activations reach four rows and four members per instruction without an LDS
+// read. (The f32 matrix rate equals the VALU's here, 117 against 110 TFLOP/s
+// measured, and they share time; what goes is the LDS traffic, 1 KB per 4 rows
+// and record piece at the 90 B/clk it is read at, and the issue slots.)
+//
+// A unit's 16 records per row reduce in canonical order: 4 lanes of a block by
+// two DPP steps, then blocks (b0 + b1) + (b2 + b3) and quarters
+// (r0 + r1) + (r2 + r3) through LDS, where the records were; one barrier per
+// kManyItems units.
+//
+// Measured (us, against rows through VALU FMAs with the records in LDS): 8
+// members, K 4096: Q4_K 4096 / 24576 / 98304 rows 10.9 / 38.3 / 134.6 -> 9.6 /
+// 30.7 / 105.4; Q5_K 24576 rows 42.7 -> 33.6; Q6_K 50.2 -> 38.7; 4 members, Q4_K
+// 24576 rows 26.1 -> 21.4. What bounds it: with the weights in cache 26.9 us, so
+// the f32 multiply-adds and the conversions; an MFMA takes 4.5 ns of a SIMD. A
+// ring of four units, two workgroups per CU (4 members), and weights loaded as
+// whole rows through an LDS slab were level or slower.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kManyWaves = 8;
+constexpr int kManyItems = 32;                     // units a wave reduces between barriers
+constexpr int kManyStride = 64 * 68 + 8;           // dwords per member's records: quads of lanes (members) in distinct banks
+constexpr int kManyLds = 4 * kManyStride * 4;      // bytes per four members
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_shift_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// part[m] = this lane's share of its row . x_m (m = 0 .. 4 MG - 1): rows_dot's
+// operation sequence per (row, member), the FMAs on the matrix cores.
+template <int T, int MG>
+__device__ __forceinline__ void unit_dot(const RowData<T>& d, int p, const float4 (&x)[MG][16], const float (&xg)[MG][4],
+                                         float (&part)[4 * MG]) {
+    constexpr int CH = 8;  // dwords of quants per run
+    auto mac = [](float xv, float q, f32x4 s) { return __builtin_amdgcn_mfma_f32_4x4x1f32(xv, q, s, 0, 0, 0); };
+    // Quants are converted in runs, then multiplied in runs: a VALU instruction
+    // between two MFMAs costs about 1 ns more than one after another VALU
+    // instruction (8 members, Q4_K 4096 -> 98304: 122 us alternating, 106 in
+    // runs of 32 quants). The minimum terms m * X run as one more MFMA each.
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (T == kQ4K || T == kQ5K) {
+        float a0, a1, b0, b1;
+        group_scales<T>(d.h, p, a0, a1, b0, b1);
+        f32x4 sA[MG], sB[MG], mA[MG], mB[MG];
+#pragma unroll
+        for (int h = 0; h < 8; h += CH) {
+            float fa[CH][4], fb[CH][4];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) quant_quads<T>(d, h + j, p, fa[j], fb[j]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < CH; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int g = 0; g < MG; ++g) {
+                        const float4 xa = x[g][h + j], xb = x[g][8 + h + j];
+                        const float va[4] = {xa.x, xa.y, xa.z, xa.w}, vb[4] = {xb.x, xb.y, xb.z, xb.w};
+                        sA[g] = mac(va[t], fa[j][t], h + j + t == 0 ? zero : sA[g]);
+                        sB[g] = mac(vb[t], fb[j][t], h + j + t == 0 ? zero : sB[g]);
+                    }
+            if (h + CH == 8) {
+#pragma unroll
+                for (int g = 0; g < MG; ++g) {
+                    mA[g] = mac(xg[g][0], b0, zero);
+                    mB[g] = mac(xg[g][1], b1, zero);
                 }
             }
-            if constexpr (ONE_SLICE) {
-                ++crow;
-            } else if (r % GROUP == GROUP - 1 && ++cslice == slices) {
-                cslice = 0;
-                crow += GROUP;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int g = 0; g < MG; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float tA = __builtin_fmaf(a0, sA[g][i], -mA[g][i]);
+                const float tB = __builtin_fmaf(a1, sB[g][i], -mB[g][i]);
+                part[4 * g + i] = tA + tB;
             }
-        };
+    } else {
+        float a[4];
+        uint32_t law[4], lbw[4], qhw[4];
+        q6_fields(d, p, a, law, lbw, qhw);
+        float acc[4 * MG];
+        // two 16-element groups at a time: their chains are independent
+#pragma unroll
+        for (int v = 0; v < 4; v += 2) {
+            f32x4 s0[MG], s1[MG], m0[MG], m1[MG];
+            constexpr int CH6 = MG == 1 ? 4 : 2;  // two groups of members leave registers for half a run
+#pragma unroll
+            for (int h = 0; h < 4; h += CH6) {
+                float f0[CH6][4], f1[CH6][4];
+#pragma unroll
+                for (int j = 0; j < CH6; ++j) {
+                    q6_quad(law[h + j], qhw[h + j], v, f0[j]);
+                    q6_quad(lbw[h + j], qhw[h + j], v + 1, f1[j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < CH6; ++j)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int g = 0; g < MG; ++g) {
+                            const float4 x0 = x[g][4 * v + h + j], x1 = x[g][4 * v + 4 + h + j];
+                            const float w0[4] = {x0.x, x0.y, x0.z, x0.w}, w1[4] = {x1.x, x1.y, x1.z, x1.w};
+                            s0[g] = mac(w0[t], f0[j][t], h + j + t == 0 ? zero : s0[g]);
+                            s1[g] = mac(w1[t], f1[j][t], h + j + t == 0 ? zero : s1[g]);
+                        }
+                if (h + CH6 == 4) {
+#pragma unroll
+                    for (int g = 0; g < MG; ++g) {  // 32 X, exact
+                        m0[g] = mac(xg[g][v], 32.0f, zero);
+                        m1[g] = mac(xg[g][v + 1], 32.0f, zero);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int g = 0; g < MG; ++g)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float t0 = a[v] * (s0[g][i] - m0[g][i]);
+                    const float t1 = a[v + 1] * (s1[g][i] - m1[g][i]);
+                    acc[4 * g + i] = ((v == 0) ? t0 : acc[4 * g + i] + t0) + t1;
+                }
+        }
+#pragma unroll
+        for (int m = 0; m < 4 * MG; ++m) part[m] = acc[m];
+    }
+}
 
-        const int rows_w = r_end - r_begin;
-        const int units = ONE_SLICE ? rows_w : (rows_w + GROUP - 1) / GROUP * GROUP * slices;
-        const int passes = (units + NBUF - 1) / NBUF;
-        for (int ps = 0; ps + 1 < passes; ++ps) {
+}  // namespace
+
+// MG: groups of four members (1: 3..4 members, 2: 5..8). SPLIT: K spans
+// several slices; the first `wgs` workgroups take slice 0, the next slice 1,
+// ..., the rest the last one (which may be short), and each row's slice total
+// P_s goes to args.partial[s][members][rows] for f32_split_reduce_kernel, and
+// with an RMSNorm the blocks' sums of squares to [members][super-blocks] after
+// the partials.
+template <int T, int MG, int PRO, int NBUF, bool PAIR, bool SPLIT>
+__global__ __launch_bounds__(kManyWaves * 64) void gemv_f32_many_kernel(WaveGemvArgs args, int wgs) {
+    static_assert(kManyItems % NBUF == 0, "whole ring passes between barriers");
+    static_assert(!PAIR || NBUF % 2 == 0, "pairs are whole ring slots");
+    static_assert(!SPLIT || !PAIR, "slice splits store slice totals");
+    constexpr bool NORM = PRO == kProNorm;
+    constexpr int MT = 4 * MG;
+    constexpr int BB = BlockTraits<T>::bytes;
+    constexpr int NBW = 16 / kManyWaves;  // staging blocks per wave
+    extern __shared__ float xs[];         // [MT][64 records][68] (member stride kManyStride), then the units' block sums
+    __shared__ float ssq_s[NORM && !SPLIT ? MT : 1][NORM && !SPLIT ? 16 : 1];
+    __shared__ float inv_s[MT];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int K = args.K;
+    const int nb = K >> 8;
+    const int members = args.members;
+    const int last_slice = (nb - 1) >> 4;
+    const int slice0 = SPLIT ? min((int)blockIdx.x / wgs, last_slice) : 0;
+    const int wg = SPLIT ? (int)blockIdx.x - slice0 * wgs : (int)blockIdx.x;
+    const int wg_count = !SPLIT ? (int)gridDim.x : slice0 < last_slice ? wgs : (int)gridDim.x - last_slice * wgs;
+    // quarters with blocks in this slice, and the sets of waves that share them out
+    const int quarters = (min(nb - 16 * slice0, 16) + 3) >> 2;
+    const int sets = quarters == 1 ? 8 : quarters == 2 ? 4 : 2;
+    const int quarter = wave % quarters;
+    const int set = wave / quarters;  // sets..: idle (three quarters use six waves)
+    const uint32_t row_bytes = (uint32_t)nb * BB;
+
+    // units of four rows, numbered through the matrices; a matrix's last one may be short
+    int unit_end[kMaxGroup];
 #pragma unroll
-            for (int r = 0; r < NBUF; ++r) {
-                consume(ring[r], r);
-                load_next(ring[r], r);
+    for (int i = 0; i < kMaxGroup; ++i) {
+        const int rows = args.rows_end[i] - (i > 0 ? args.rows_end[i - 1] : 0);
+        unit_end[i] = (i > 0 ? unit_end[i - 1] : 0) + (i < args.count ? (rows + 3) >> 2 : 0);
+    }
+    const int units = PAIR ? unit_end[0] : unit_end[kMaxGroup - 1];
+    const int u_begin = (int)((long long)units * wg / wg_count);
+    const int u_end = (int)((long long)units * (wg + 1) / wg_count);
+    // this wave's item k: unit u_begin + set + sets * k (pairs: gate rows for even k, up rows of the same unit for odd k)
+    const int items = (PAIR ? 2 : 1) * ((u_end - u_begin + sets - 1) / sets);
+    auto unit_of = [&](int s, int k) { return u_begin + s + sets * (PAIR ? k >> 1 : k); };
+    auto locate = [&](int unit, int k, int& mat, int& row0) {
+        mat = 0;
+        int start = 0;
+        if constexpr (PAIR) {
+            mat = k & 1;
+        } else {
+#pragma unroll
+            for (int i = 0; i < kMaxGroup - 1; ++i) {
+                if (i + 1 < args.count && unit >= unit_end[i]) {
+                    mat = i + 1;
+                    start = unit_end[i];
+                }
             }
         }
-        if (passes > 0) {
-            const int left = units - (passes - 1) * NBUF;
+        row0 = 4 * (unit - start);
+    };
+
+    // ---- activation loads first, then the first units of weights, then the
+    // staging (vector memory returns in order)
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(args.x, (uint32_t)members * (uint32_t)K * 4u);
+    const __amdgpu_buffer_rsrc_t gr = make_rsrc(args.gamma, NORM ? (uint32_t)K * 4u : 0u);
+    float4 xv[NBW][MT];
+    float4 gv[NORM ? NBW : 1];
 #pragma unroll
-            for (int r = 0; r < NBUF; ++r) {
-                if (r < left) consume(ring[r], r);
+    for (int k = 0; k < NBW; ++k) {
+        const int b = 16 * slice0 + wave + kManyWaves * k;
+        const int e = 256 * b + 4 * lane;
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            xv[k][m] = load_f4(xr, (b < nb && m < members) ? (uint32_t)(m * K + e) * 4u : kOutOfRange);
+        if constexpr (NORM) gv[k] = load_f4(gr, b < nb ? (uint32_t)e * 4u : kOutOfRange);
+    }
+    asm volatile("" ::: "memory");
+
+    const int slot = lane >> 2;      // record of the quarter
+    const int p = slot & 3;          // quarter of its super-block
+    const int block = 16 * slice0 + 4 * quarter + (slot >> 2);
+    const uint32_t lane_off = (uint32_t)(lane & 3) * row_bytes + (uint32_t)block * BB;
+    RowData<T> ring[NBUF];
+    auto load_item = [&](RowData<T>& dst, int k) {
+        const int unit = unit_of(set, k);
+        int mat, row0;
+        locate(unit, k, mat, row0);
+        const uint8_t* w = args.w[0];
+        uint32_t bytes = args.wbytes[0];
+#pragma unroll
+        for (int i = 1; i < kMaxGroup; ++i) {
+            if (mat == i) {
+                w = args.w[i];
+                bytes = args.wbytes[i];
             }
         }
+        // dead items read through an empty resource; rows past the matrix lie
+        // past its bytes: zeros
+        const bool live = set < sets && unit < u_end;
+        load_row<T>(dst, make_rsrc(w, live ? bytes : 0u), block < nb ? lane_off + (uint32_t)row0 * row_bytes : kOutOfRange, p);
+    };
+#pragma unroll
+    for (int r = 0; r < NBUF; ++r) load_item(ring[r], r);
+
+#pragma unroll
+    for (int k = 0; k < NBW; ++k) {
+        const int b = 16 * slice0 + wave + kManyWaves * k;
+        int rec, pos;
+        f32_slot<T>(256 * (b - 16 * slice0) + 4 * lane, rec, pos);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            float4 v = xv[k][m];
+            if constexpr (NORM) {
+                const float sq = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+                const float blk = wave_sum_uniform(sq);
+                if (lane == 0 && b < nb && m < members) {
+                    if constexpr (SPLIT) {
+                        if (wg == 0)
+                            args.partial[(size_t)(last_slice + 1) * members * args.total_rows + (size_t)m * nb + b] = blk;
+                    } else {
+                        ssq_s[m][b] = blk;
+                    }
+                }
+                v.x *= gv[k].x;
+                v.y *= gv[k].y;
+                v.z *= gv[k].z;
+                v.w *= gv[k].w;
+            }
+            const float gsum = group_sum_f<T>(((v.x + v.y) + v.z) + v.w);
+            // blocks past K are staged as zeros, absent members' too
+            float* dst = xs + m * kManyStride + rec * F32Rec<T>::stride;
+            *reinterpret_cast<float4*>(dst + pos) = v;
+            if ((lane & (F32Rec<T>::group / 4 - 1)) == 0) dst[64 + pos / F32Rec<T>::group] = gsum;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < MT) {
+        float inv = 1.f;
+        if constexpr (NORM && !SPLIT) {
+            if ((int)threadIdx.x < members) {
+                float total = 0.f;
+                for (int b = 0; b < nb; ++b) total += ssq_s[threadIdx.x][b];
+                // RMSNorm (qwen_reference.rs:550-556): x * (1/sqrt(sum(x^2)/K + eps)) * gamma
+                inv = 1.0f / sqrtf(total / (float)K + args.eps);
+            }
+        }
+        inv_s[threadIdx.x] = inv;
+    }
+    float4 x[MG][16];
+    float xg[MG][4];
+#pragma unroll
+    for (int g = 0; g < MG; ++g) {
+        const float* src = xs + (4 * g + (lane & 3)) * kManyStride + (16 * quarter + slot) * F32Rec<T>::stride;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[g][i] = *reinterpret_cast<const float4*>(src + 4 * i);
+        const float4 sums = *reinterpret_cast<const float4*>(src + 64);
+        xg[g][0] = sums.x;
+        xg[g][1] = sums.y;
+        xg[g][2] = sums.z;
+        xg[g][3] = sums.w;
+    }
+    __syncthreads();
+
+    // block sums: [item][wave][block of the quarter][row of the unit][member]
+    constexpr int kWaveSums = 16 * MT;
+    constexpr int kItemSums = kManyWaves * kWaveSums;
+    static_assert((size_t)kManyItems * kItemSums * 4 <= (size_t)MG * kManyLds, "block sums fit the records' room");
+    const __amdgpu_buffer_rsrc_t partial_r =
+        make_rsrc(args.partial, SPLIT ? (uint32_t)(last_slice + 1) * (uint32_t)members * (uint32_t)args.total_rows * 4u : 0u);
+
+    // The rows of items [first, first + count): value v = (item, set, row of
+    // the unit, member), the members fastest.
+    auto finish = [&](int first, int count) {
+        const int values = (PAIR ? count >> 1 : count) * sets * (4 * MT);
+        for (int v = threadIdx.x; v < values; v += kManyWaves * 64) {
+            const int m = v % MT, j = (v / MT) & 3;
+            const int s = (v / (4 * MT)) & (sets - 1);
+            const int item = (v / (4 * MT) / sets) * (PAIR ? 2 : 1);
+            auto total_of = [&](int it) {
+                float r[4] = {0.f, 0.f, 0.f, 0.f};
+                const float* src = xs + it * kItemSums + s * quarters * kWaveSums + j * MT + m;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (q < quarters)
+                        r[q] = (src[q * kWaveSums] + src[q * kWaveSums + 4 * MT]) +
+                               (src[q * kWaveSums + 8 * MT] + src[q * kWaveSums + 12 * MT]);
+                return (r[0] + r[1]) + (r[2] + r[3]);
+            };
+            const int unit = unit_of(s, first + item);
+            int mat, row0;
+            locate(unit, PAIR ? 0 : first + item, mat, row0);
+            const int begin = mat > 0 ? args.rows_end[mat - 1] : 0;
+            const int rows = args.rows_end[mat] - begin;
+            const int row = row0 + j;
+            if (unit >= u_end || row >= rows || m >= members) continue;
+            const float total = total_of(item);
+            if constexpr (SPLIT) {
+                const uint32_t off = (uint32_t)((slice0 * members + m) * args.total_rows + begin + row) * 4u;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, total), partial_r, (int)off, 0, 0);
+            } else {
+                float* y = args.y[0];
+#pragma unroll
+                for (int i = 1; i < kMaxGroup; ++i)
+                    if (mat == i) y = args.y[i];
+                float value = total * inv_s[m];
+                if constexpr (PAIR) {
+                    // silu(gate) * up (model_ops.rs:316-328)
+                    const float up = total_of(item + 1) * inv_s[m];
+                    value = (value / (1.0f + expf(-value))) * up;
+                }
+                float* dst = y + (size_t)m * rows + row;
+                if (args.accumulate) {
+                    unsafeAtomicAdd(dst, value);
+                } else {
+                    *dst = value;
+                }
+            }
+        }
+    };
+
+    for (int c0 = 0; c0 < items; c0 += kManyItems) {
+        const int count = min(kManyItems, items - c0);
+        for (int k0 = 0; k0 < count; k0 += NBUF) {
+#pragma unroll
+            for (int r = 0; r < NBUF; ++r) {
+                float part[MT];
+                unit_dot<T, MG>(ring[r], p, x, xg, part);
+                load_item(ring[r], c0 + k0 + r + NBUF);
+                // a block's four records: ((0 + 1) + (2 + 3)), in the block's first quad
+#pragma unroll
+                for (int m = 0; m < MT; ++m) part[m] = dpp_shift_add<0x108>(dpp_shift_add<0x104>(part[m]));  // row_shl 4, 8
+                if ((lane & 12) == 0 && set < sets) {
+                    float* dst = xs + (k0 + r) * kItemSums + wave * kWaveSums + (4 * (lane >> 4) + (lane & 3)) * MT;
+#pragma unroll
+                    for (int g = 0; g < MG; ++g)
+                        *reinterpret_cast<float4*>(dst + 4 * g) =
+                            float4{part[4 * g], part[4 * g + 1], part[4 * g + 2], part[4 * g + 3]};
+                }
+            }
+        }
+        __syncthreads();
+        finish(c0, count);
+        __syncthreads();
     }
 }
 
@@ -786,14 +1026,27 @@ template <int T, int MT, int PRO, bool ONE_SLICE, int NBUF, int WAVES, int GROUP
 std::atomic<int> F32Instance<T, MT, PRO, ONE_SLICE, NBUF, WAVES, GROUP, PAIR, SPLIT>::occupancy{0};
 
 // y[m][row] (+)= ((P_0 + P_1) + P_2) ... over the slices of a SPLIT launch,
-// in slice order: the slice totals of the one-launch form, added the same way.
+// in slice order, times the RMSNorm factor: the slice totals of the one-launch
+// form, added the same way.
 __global__ __launch_bounds__(256) void f32_split_reduce_kernel(WaveGemvArgs a, int slices) {
     const int total = a.members * a.total_rows;
+    __shared__ float inv_s[kWaveMaxMembers];
+    if (a.gamma != nullptr) {
+        const int nb = a.K >> 8;
+        if ((int)threadIdx.x < a.members) {
+            const float* ssq = a.partial + (size_t)slices * total + (size_t)threadIdx.x * nb;
+            float sum = 0.f;
+            for (int b = 0; b < nb; ++b) sum += ssq[b];
+            inv_s[threadIdx.x] = 1.0f / sqrtf(sum / (float)a.K + a.eps);
+        }
+        __syncthreads();
+    }
     for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
         const int m = i / a.total_rows;
         const int row = i - m * a.total_rows;
         float t = a.partial[(size_t)m * a.total_rows + row];
         for (int s = 1; s < slices; ++s) t = t + a.partial[((size_t)s * a.members + m) * a.total_rows + row];
+        if (a.gamma != nullptr) t = t * inv_s[m];
         int mat = 0, start = 0;
         for (int g = 0; g + 1 < a.count; ++g) {
             if (row >= a.rows_end[g]) {
@@ -836,12 +1089,39 @@ hipError_t launch_few(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
     }
 }
 
-// Three to eight members, one slice.
-template <int T, int PRO, bool PAIR>
+// Three to eight members (one form for all: at three, 4-member groups still beat
+// the VALU rows, 6.6 against 7.5 us at 4096 rows): one workgroup per CU over the slice (or, SPLIT, over
+// the slices in proportion to their super-blocks).
+template <int T, int MG, int PRO, bool PAIR, bool SPLIT = false>
+hipError_t launch_many_instance(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
+    constexpr int kRing = 2;
+    auto kern = gemv_f32_many_kernel<T, MG, PRO, kRing, PAIR, SPLIT>;
+    static std::atomic<bool> sized{false};
+    if (!sized.load(std::memory_order_relaxed)) {
+        const hipError_t e =
+            hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, MG * kManyLds);
+        if (e != hipSuccess) return e;
+        sized.store(true, std::memory_order_relaxed);
+    }
+    const int nb = a.K >> 8;
+    const int slices = SPLIT ? (nb + 15) >> 4 : 1;
+    long long units = 0;
+    for (int i = 0; i < (PAIR ? 1 : a.count); ++i)
+        units += (a.rows_end[i] - (i > 0 ? a.rows_end[i - 1] : 0) + 3) / 4;
+    // workgroups of a whole slice, and of the last one (its share of the quarters)
+    const int quarters = (nb + 3) >> 2, last = quarters - 4 * (slices - 1);
+    const int sets = last == 1 ? 8 : last == 2 ? 4 : 2;
+    const int wgs = (int)std::max<long long>(1, std::min<long long>((units + 1) / 2, (long long)cu_count * (slices == 1 ? last : 4) / quarters));
+    const int tail = (int)std::max<long long>(1, std::min<long long>((units + sets - 1) / sets, cu_count - (long long)wgs * (slices - 1)));
+    const int grid = slices == 1 ? tail : wgs * (slices - 1) + tail;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kManyWaves * 64), MG * kManyLds, stream, a, wgs);
+    return hipGetLastError();
+}
+
+template <int T, int PRO, bool PAIR, bool SPLIT = false>
 hipError_t launch_many(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
-    if (a.members <= 4) return F32Instance<T, 4, PRO, true, 4, 8, 1, PAIR>::launch(a, cu_count, 1, stream);
-    // ring depth: 4 rows where the registers allow (Q6_K rows need 22 VGPRs)
-    return F32Instance<T, 8, PRO, true, (T != kQ6K ? 4 : PAIR ? 2 : 3), 8, 1, PAIR>::launch(a, cu_count, 1, stream);
+    return a.members <= 4 ? launch_many_instance<T, 1, PRO, PAIR, SPLIT>(a, cu_count, stream)
+                          : launch_many_instance<T, 2, PRO, PAIR, SPLIT>(a, cu_count, stream);
 }
 
 template <int T, int PRO>
@@ -893,10 +1173,8 @@ template <int T>
 hipError_t launch_split(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
     hipError_t e = (a.members == 1)
                        ? F32Instance<T, 1, kProPlain, true, 3, 8, 1, false, true>::launch(a, cu_count, 1, stream)
-                   : (a.members <= 4)
-                       ? F32Instance<T, 4, kProPlain, true, 4, 8, 1, false, true>::launch(a, cu_count, 1, stream)
-                       : F32Instance<T, 8, kProPlain, true, (T != kQ6K ? 4 : 3), 8, 1, false, true>::launch(
-                             a, cu_count, 1, stream);
+                   : a.gamma != nullptr ? launch_many<T, kProNorm, false, true>(a, cu_count, stream)
+                                        : launch_many<T, kProPlain, false, true>(a, cu_count, stream);
     if (e != hipSuccess) return e;
     const int slices = ((a.K >> 8) + 15) >> 4;
     const long long total = (long long)a.members * a.total_rows;
@@ -915,9 +1193,9 @@ size_t f32_split_partial_bytes(int members, int K, int total_rows) {
 hipError_t launch_gemv_f32_split(int value_type, const WaveGemvArgs& args, int cu_count, hipStream_t stream) {
     const int min_members = args.K > kWaveMaxK ? 1 : 3;
     if (args.members < min_members || args.members > kWaveMaxMembers || args.K <= kSliceElems ||
-        args.K > kF32SplitMaxK || args.K % 256 != 0 || args.gamma != nullptr || args.x2 != nullptr ||
+        args.K > kF32SplitMaxK || args.K % 256 != 0 || (args.gamma != nullptr && args.members < 3) || args.x2 != nullptr ||
         args.pair_swiglu || args.partial == nullptr ||
-        f32_split_partial_bytes(args.members, args.K, args.total_rows) > kF32SplitScratchBytes) {
+        f32_split_partial_bytes(args.members, args.K, args.total_rows) > (args.K > kWaveMaxK ? kF32SplitScratchBytes : kF32MmaPartialBytes)) {
         return hipErrorInvalidValue;
     }
     switch (value_type) {

@@ -768,9 +768,9 @@ hipError_t launch_gemv(int value_type, const WaveGemvArgs& a0, void* act_scratch
         int per = f32_max_members(a.K);
         if (a.x2 != nullptr) per = std::min(per, kSwigluMaxMembers);
         if (per <= 0) return hipErrorInvalidValue;
-        const bool splittable = a.K > kSliceK && a.x2 == nullptr && a.gamma == nullptr && !a.pair_swiglu &&
+        const bool splittable = a.K > kSliceK && a.x2 == nullptr && !a.pair_swiglu &&
                                 act_scratch != nullptr &&
-                                f32_split_partial_bytes(kWaveMaxMembers, a.K, a.total_rows) <= kF32SplitScratchBytes;
+                                f32_split_partial_bytes(kWaveMaxMembers, a.K, a.total_rows) <= kF32MmaPartialBytes;
         if (splittable) per = kWaveMaxMembers;
         for (int m0 = 0; m0 < a.members; m0 += per) {
             WaveGemvArgs c = a;

@@ -680,3 +680,40 @@ def test_random_shapes_fused_rms_norm(env, mode, i, t, k, n, members):
     for m in sorted({0, members // 2, members - 1}):
         normed = O.rms_norm_raw(x[m], gam, 1e-6)
         assert max_rel_err(got[m], O.quant_gemv(t, enc, k, n, normed, threads=16)) <= RTOL
+
+
+@pytest.mark.parametrize("t,blocks,ns,members,norm", [
+    (12, 1, (4, 1, 7), 3, True), (13, 3, (1030,), 8, False), (14, 4, (63,), 5, True), (12, 5, (2049, 2), 8, True),
+    (14, 9, (37, 301), 4, False), (13, 13, (515,), 7, True), (12, 16, (66000,), 8, False), (14, 16, (4099,), 6, True),
+    (12, 17, (129, 3), 8, True), (13, 20, (1001,), 3, False), (14, 20, (77,), 8, True), (12, 33, (263,), 6, True),
+    (12, 64, (19,), 4, True)])
+def test_many_members_edges_bit_identical(env, t, blocks, ns, members, norm):
+    """3..8 members at the edges of the f32 matrix-core form: one to four quarters of a slice
+    (4 super-blocks each) and partial ones, short last units of four rows in each matrix of a
+    group, more units than one barrier interval, several slices (with the RMSNorm factor applied
+    after the slice sum): every row bit-identical to its single-member call, member 0 and the last
+    within the f32 bar of the oracle, and the accumulating form equal to a store plus an add."""
+    k = 256 * blocks
+    print_case(test="many_edges", t=t, k=k, ns=ns, members=members, norm=norm)
+    encs = [synth.kquant_numpy(t, k, n, seed=k + n + j) for j, n in enumerate(ns)]
+    ws = [upload(env, t, k, n, e) for n, e in zip(ns, encs)]
+    x = synth.activations_numpy(k, members, seed=31 * blocks + members)
+    gamma = synth.gamma_numpy(k, seed=blocks)
+    kern = env["k"][t]
+    g = to_dev(gamma) if norm else None
+    ys = [empty_dev(members * n) for n in ns]
+    kern.execute_group(ws, to_dev(x.reshape(-1)), ys, members, gamma=g, epsilon=1e-6)
+    for w, n, enc, y in zip(ws, ns, encs, ys):
+        got = to_host(y, env["ctx"]).reshape(members, n)
+        for m in range(members):
+            y1 = empty_dev(n)
+            kern.execute_group([w], to_dev(x[m]), [y1], 1, gamma=g, epsilon=1e-6)
+            assert np.array_equal(to_host(y1, env["ctx"]).view(np.uint32), got[m].view(np.uint32)), m
+        for m in {0, members - 1}:
+            xin = O.rms_norm_raw(x[m], gamma, 1e-6) if norm else x[m]
+            assert max_rel_err(got[m], O.quant_gemv(t, enc, k, n, xin, threads=8)) <= F32_RTOL
+    base = synth.activations_numpy(ns[0], members, seed=3).reshape(-1)
+    acc = to_dev(base)
+    kern.execute_fused(ws[0], to_dev(x.reshape(-1)), acc, members, gamma=g, epsilon=1e-6, accumulate=True)
+    want = base + to_host(ys[0], env["ctx"])
+    assert np.array_equal(to_host(acc, env["ctx"]).view(np.uint32), want.view(np.uint32))

@@ -912,6 +912,421 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
     }
 }
 
+// attn_prefill_wide_kernel: causal attention of a prompt chunk on the matrix cores
+// (v_mfma_f32_32x32x16_f16, f32 accumulation), after kv_append_seq_kernel
+// stored the chunk's K/V. Token t (position p0 + t) attends positions
+// 0 .. p0 + t: the reference's attention (model_ops.rs:430-566) for every
+// token of the chunk, as the serial prefill computes it one token at a time.
+//
+// The form for many tokens (wide_prefill); the arithmetic is attn_prefill_kernel's.
+// A wave owns one query head and kPrefillWideTokens (32) tokens; a workgroup
+// holds the QPK query heads of one KV head (and, for QPK < 4, 4 / QPK token
+// tiles), so every K/V byte it stages serves all of them, and every byte a
+// wave reads from LDS serves 32 tokens: 64 B per CU and clock of reads under
+// the MFMAs, against 128 with 16 tokens, which is more than LDS delivers (90).
+// Keys advance in blocks of 64 through double-buffered LDS as there; V^T rows are
+// 72 halfs for 16-byte reads (the 8 lanes of an LDS cycle fall in distinct
+// banks).
+//
+// Per block and wave, with S^T = K Q^T (M = 32 keys, N = 32 tokens, K = 128
+// dims in 8 steps) the MFMA output puts token l%32 in lane l's column and keys
+// 8(i/4) + 4(l/32) + i%4 in its 16 rows, so the online softmax state of a
+// token lives in its two lanes. The probabilities are already the B operand of
+// O^T += V^T P^T (M = 32 dims, K = 16 keys): a dot product does not depend on
+// the order of its terms, so key slot 8h+j of a 16-key step is key 4h + 8(j/4)
+// + j%4, and V^T stores a step's keys in that order (vt_pos).
+//
+// Two key halves: eight waves, four of which take the even key blocks and four
+// the odd ones, meeting through LDS at the end (QPK = 8 fills eight waves with
+// its heads). The longest causal range sets the launch's time, and a wave alone
+// on its SIMD takes 2.5 us a block, two together little more.
+//
+// Workgroups: one per CU, longest causal ranges first; KV head fastest (with 8
+// of them, one per XCD, whose L2 then holds that head's K/V).
+//
+// Measured, 2,047 tokens of 32 / 8 heads: 127-133 -> 88 us (kernel), of which 66
+// are the key rounds (1.1 PFLOP/s of issued MFMAs; without the lo products 44,
+// without the staging 62). A round takes 2.6 us with few CUs busy and 3.9 with
+// all of them: the clock under load, not a stall, and about what the library's
+// dense products reach (1.17 PFLOP/s).
+typedef float pf_float16 __attribute__((ext_vector_type(16)));
+
+constexpr int kPfWideVRow = kPfKeys + 8;     // LDS V^T row (halfs): 144 B
+// Instruction classes of __builtin_amdgcn_sched_group_barrier.
+constexpr int kSchedValu = 0x2, kSchedMfma = 0x8, kSchedLdsRead = 0x100;
+
+// Where V^T keeps key k of a block (k a multiple of 4: four keys stay together).
+__device__ __forceinline__ int vt_pos(int k) { return (k & ~15) | ((k & 4) << 1) | ((k & 8) >> 1); }
+
+// The value of lane ^ 32 combined into both lanes. (The halves are copied out
+// before the bit casts: a cast of a vector element reads element 0.)
+template <class OP>
+__device__ __forceinline__ float pair_combine(float v, OP op) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    const uint32_t lo = r[0], hi = r[1];
+    return op(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+
+template <int QPK>
+__global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnArgs a, int tiles) {
+    constexpr int KS = QPK < 8 ? 2 : 1;   // key halves
+    constexpr int W = 8 / KS;             // waves per key half
+    constexpr int NT = 64 * W;
+    constexpr int TT = W / QPK;           // token tiles per workgroup
+    constexpr int TOK = kPrefillWideTokens;
+    constexpr int KP = kPfKeys * (kHeadDim / 8) / NT;  // 16-byte K pieces per thread and block
+    // V: 256 units of 4 keys x 8 dims, one per thread of a half's first 256
+    struct Buffer {
+        _Float16 k[kPfKeys][kHeadDim];
+        _Float16 v[kHeadDim][kPfWideVRow];
+    };
+    // before the key loop the room holds the query pieces and the rope table
+    constexpr int kRows = 128;                        // (token, head) rows of query pieces at a time
+    constexpr int kRotRow = 65;                       // float2 per token row (padded)
+    constexpr int kQBytes = kRows * kHeadDim * 2 * 2;  // hi and lo
+    constexpr int kPrologue = kQBytes + TT * TOK * kRotRow * 8;
+    constexpr int kLoop = 2 * KS * (int)sizeof(Buffer);
+    __shared__ __attribute__((aligned(16))) char lds[kLoop > kPrologue ? kLoop : kPrologue];
+    Buffer(*const bufs)[KS] = reinterpret_cast<Buffer(*)[KS]>(lds);
+
+    const int tid = threadIdx.x & (NT - 1);
+    const int lane = tid & 63;
+    const int half = __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // of its key half
+    const int kvh = (int)blockIdx.x % a.kv_heads;
+    const int tile = tiles - 1 - (int)blockIdx.x / a.kv_heads;
+    const int hq = kvh * QPK + wave % QPK;
+    const int t0 = (tile * TT + wave / QPK) * TOK;
+    const int tl = lane & 31;
+    const int h = lane >> 5;
+    const int t = t0 + tl;
+    const bool live = t < a.tokens;
+    const int pos = a.p0 + t;
+    const int qdim = a.q_heads * kHeadDim;
+    // the last position any token of the workgroup attends
+    const int wg_end = min((tile + 1) * TT * TOK, a.tokens);
+    const int last = a.p0 + wg_end - 1;
+
+    // ---- K/V block loads (positions past `last` read as zero)
+    const size_t head_elems = (size_t)a.mem.capacity * kHeadDim;
+    const size_t base = (size_t)a.layer * a.mem.layer_elems + (size_t)kvh * head_elems;
+    const uint32_t span = (uint32_t)(last + 1) * (uint32_t)(kHeadDim * 2);
+    const __amdgpu_buffer_rsrc_t kr = make_rsrc(a.mem.keys + base, span);
+    const __amdgpu_buffer_rsrc_t vr = make_rsrc(a.mem.values + base, span);
+    const bool v_unit = tid < 256;
+    const int va = tid & 15;        // V unit: keys 4va .. 4va + 3
+    const int vc = (tid >> 4) & 15; // dims 8vc .. 8vc + 7
+    auto issue_k = [&](int kb, uint4 (&kp)[KP]) {
+#pragma unroll
+        for (int r = 0; r < KP; ++r) {
+            const int idx = tid + NT * r;
+            kp[r] = load_b128(kr, ((uint32_t)(kb * kPfKeys + (idx >> 4)) * kHeadDim + 8u * (uint32_t)(idx & 15)) * 2u);
+        }
+    };
+    auto stage_k = [&](int buf, const uint4 (&kp)[KP]) {
+#pragma unroll
+        for (int r = 0; r < KP; ++r) {
+            const int idx = tid + NT * r;
+            *reinterpret_cast<uint4*>(&bufs[buf][half].k[idx >> 4][8 * ((idx & 15) ^ ((idx >> 4) & 15))]) = kp[r];
+        }
+    };
+    auto issue_v = [&](int kb, uint4 (&vp)[4]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t off = ((uint32_t)(kb * kPfKeys + 4 * va + r) * kHeadDim + 8u * (uint32_t)vc) * 2u;
+            vp[r] = load_b128(vr, v_unit ? off : kOOR);
+        }
+    };
+    auto stage_v = [&](int buf, const uint4 (&vp)[4]) {
+        if (v_unit) {
+            // row j of the unit: dim 8vc + j of keys 4va .. 4va + 3
+            const uint32_t w[4][4] = {{vp[0].x, vp[0].y, vp[0].z, vp[0].w}, {vp[1].x, vp[1].y, vp[1].z, vp[1].w},
+                                      {vp[2].x, vp[2].y, vp[2].z, vp[2].w}, {vp[3].x, vp[3].y, vp[3].z, vp[3].w}};
+            const int at = vt_pos(4 * va);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                // halfword j & 1 of words j >> 1 of two keys, packed by one byte permute each
+                const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+                const uint32_t e01 = __builtin_amdgcn_perm(w[1][j >> 1], w[0][j >> 1], sel);
+                const uint32_t e23 = __builtin_amdgcn_perm(w[3][j >> 1], w[2][j >> 1], sel);
+                *reinterpret_cast<uint2*>(&bufs[buf][half].v[8 * vc + j][at]) = make_uint2(e01, e23);
+            }
+        }
+    };
+
+    // ---- the prologue's loads, all in flight under the rope angles: the first
+    // K/V blocks and the query rows of the first pass (thread: 8 dims of rows
+    // tid/16 + 32 i)
+    uint4 kp0[KP], vp0[4];
+    issue_k(half, kp0);
+    issue_v(half, vp0);
+    const int c = threadIdx.x & 15;
+    const int r0 = (int)threadIdx.x >> 4;
+    float4 raw[kRows / 32][2];
+    auto load_rows = [&](int pass) {
+#pragma unroll
+        for (int i = 0; i < kRows / 32; ++i) {
+            const int r = r0 + 32 * i;
+            const int unit = pass * (kRows / TOK) + r / TOK;  // wave of a key half: (token tile, head)
+            const int token = (tile * TT + unit / QPK) * TOK + (r & (TOK - 1));
+            raw[i][0] = raw[i][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (token < a.tokens) {
+                const float4* src = reinterpret_cast<const float4*>(a.q + (size_t)token * qdim + (size_t)(kvh * QPK + unit % QPK) * kHeadDim + 8 * c);
+                raw[i][0] = src[0];
+                raw[i][1] = src[1];
+            }
+        }
+    };
+    load_rows(0);
+    const float4 wn[2] = {reinterpret_cast<const float4*>(a.q_norm + 8 * c)[0], reinterpret_cast<const float4*>(a.q_norm + 8 * c)[1]};
+
+    // ---- rope angles of the workgroup's tokens: entry (row, d) = the rotation
+    // of pair (d, d + 64) at position p0 + first token + row, the rope_rot /
+    // rope_freq values of the decode kernel
+    float2* const rot_tab = reinterpret_cast<float2*>(lds + kQBytes);
+    const float freq = rope_freq(a.rope_base, lane);
+#pragma unroll 1
+    for (int r = (int)threadIdx.x >> 6; r < TT * TOK; r += 8) {
+        const Rot rr = rope_rot((float)(a.p0 + tile * TT * TOK + r), freq);
+        rot_tab[r * kRotRow + lane] = make_float2(rr.c, rr.s);
+    }
+    __syncthreads();
+
+    // ---- query pieces: row (token tile, head, token of the tile), RMSNorm
+    // over the head's 128 dims, NEOX rope of the pairs (d, d + 64), f16 hi and
+    // lo. Sixteen lanes a row, eight dims each, in a short loop: a launch
+    // fetches its code cold, and unrolled per wave this took 10 us more.
+    // 16-byte piece c of row r at slot c ^ (r & 15).
+    pf_half8* const q_hi = reinterpret_cast<pf_half8*>(lds);
+    pf_half8* const q_lo = q_hi + kRows * 16;
+    pf_half8 qb[8], ql[8];
+    constexpr int kPasses = TT * TOK * QPK / kRows;
+#pragma unroll 1
+    for (int pass = 0; pass < kPasses; ++pass) {
+        if (pass > 0) load_rows(pass);
+        // a thread's own slots hold its row pieces first, then what it makes of them
+#pragma unroll
+        for (int i = 0; i < kRows / 32; ++i) {
+            const int slot = (r0 + 32 * i) * 16 + (c ^ ((r0 + 32 * i) & 15));
+            reinterpret_cast<float4*>(q_hi)[slot] = raw[i][0];
+            reinterpret_cast<float4*>(q_lo)[slot] = raw[i][1];
+        }
+#pragma unroll 1
+        for (int r = r0; r < kRows; r += 32) {
+            const int unit = pass * (kRows / TOK) + r / TOK;
+            const int slot = r * 16 + (c ^ (r & 15));
+            const float4 lo = reinterpret_cast<const float4*>(q_hi)[slot], hi = reinterpret_cast<const float4*>(q_lo)[slot];
+            const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            const float w[8] = {wn[0].x, wn[0].y, wn[0].z, wn[0].w, wn[1].x, wn[1].y, wn[1].z, wn[1].w};
+            float ssq = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ssq = __builtin_fmaf(x[j], x[j], ssq);
+            ssq = dpp_step<0xb1>(ssq);   // quad_perm [1,0,3,2]
+            ssq = dpp_step<0x4e>(ssq);   // quad_perm [2,3,0,1]
+            ssq = dpp_step<0x141>(ssq);  // row_half_mirror
+            ssq = dpp_step<0x140>(ssq);  // row_mirror
+            const float inv = 1.0f / sqrtf(ssq / (float)kHeadDim + a.eps);
+            const float2* rot = rot_tab + ((unit / QPK) * TOK + (r & (TOK - 1))) * kRotRow + 8 * (c & 7);
+            pf_half8 vh, vl;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float y = x[j] * inv * w[j];
+                const float other = __builtin_bit_cast(  // dim d +- 64: lane c ^ 8 (row_ror 8)
+                    float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0x128, 0xf, 0xf, false));
+                const float2 cs = rot[j];
+                const float q = y * cs.x + (c < 8 ? -other : other) * cs.y;
+                vh[j] = (_Float16)q;
+                vl[j] = (_Float16)(q - (float)vh[j]);
+            }
+            q_hi[slot] = vh;
+            q_lo[slot] = vl;
+        }
+        __syncthreads();
+        if (kPasses == 1 || wave / (kRows / TOK) == pass) {
+            // this lane's dims 16s + 8h + j of its token
+            const int r = (wave % (kRows / TOK)) * TOK + tl;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                qb[s] = q_hi[r * 16 + ((2 * s + h) ^ (r & 15))];
+                ql[s] = q_lo[r * 16 + ((2 * s + h) ^ (r & 15))];
+            }
+        }
+        __syncthreads();
+    }
+
+    // ---- online softmax over the key blocks
+    float m_run = -FLT_MAX, l_run = 0.f;
+    pf_float16 o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
+    // key half `half` takes blocks half, half + KS, ...; a block past the last
+    // is wholly masked (its loads read zeros)
+    const int rounds = (last / kPfKeys + KS) / KS;
+    stage_k(0, kp0);
+    stage_v(0, vp0);
+    __syncthreads();
+    for (int round = 0; round < rounds; ++round) {
+        const int kb = KS * round + half;
+        const int buf = round & 1;
+        // the next block: K in flight under the scores, V under the
+        // probabilities and the outputs (each held alone: registers)
+        uint4 kp[KP], vp[4];
+        if (round + 1 < rounds) issue_k(kb + KS, kp);
+
+        // S^T for the block's two 32-key tiles, interleaved: consecutive MFMAs
+        // feed different accumulators
+        pf_float16 sc[2];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[kt][i] = 0.f;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            pf_half8 ka[2];
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+                ka[kt] = *reinterpret_cast<const pf_half8*>(&bufs[buf][half].k[32 * kt + tl][8 * ((2 * s + h) ^ (tl & 15))]);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[kt], qb[s], sc[kt], 0, 0, 0);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[kt], ql[s], sc[kt], 0, 0, 0);
+        }
+        // fragment reads two steps ahead of their MFMAs
+        __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 4, 0);
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 2, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 8, 0);
+        // into the other buffer: every wave finished reading it before the
+        // previous barrier
+        if (round + 1 < rounds) {
+            stage_k(buf ^ 1, kp);
+            issue_v(kb + KS, vp);
+        }
+        // keys past a token's position are masked; a block wholly at or below
+        // the wave's first position needs no mask (a wave-uniform test)
+        if (kb * kPfKeys + kPfKeys - 1 > a.p0 + t0) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key = kb * kPfKeys + 32 * kt + 8 * (i >> 2) + 4 * h + (i & 3);
+                    if (key > pos) sc[kt][i] = -INFINITY;
+                }
+            }
+        }
+        float bmax = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) bmax = fmaxf(bmax, sc[kt][i]);
+        bmax = pair_combine(bmax, [](float u, float v) { return fmaxf(u, v); }) * a.scale;  // (scale > 0)
+        // Lazy rescaling: the reference point m_run moves (to the block's
+        // maximum) only when that maximum passes it by more than kPfLazy.
+        // Until then the probabilities exp2(s - m_run) stay below
+        // 2^kPfLazy, inside f16 range for the hi/lo split, and O and l keep
+        // their scale; O / l is the same softmax. The first block always
+        // moves it (from -FLT_MAX, with a zero correction).
+        const bool move = bmax > m_run + kPfLazy;
+        if (__any(move)) {
+            const float m_new = move ? bmax : m_run;
+            const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new;
+            l_run *= corr;
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o[d][i] *= corr;
+        }
+        // Per 16-key step: probabilities in pairs, hi = f16(p) and lo =
+        // f16(p - hi), each pair converted by one packed instruction (round
+        // toward zero: hi + lo still carries 22 bits of p, since p - hi is
+        // exact in f32), then O^T += V^T P^T, dim tiles interleaved
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            pf_half8 pb, pl;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const int i = 8 * (u & 1) + j;
+                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u >> 1][i], a.scale, -m_run));
+                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u >> 1][i + 1], a.scale, -m_run));
+                l_run += p0;
+                l_run += p1;
+                const auto hi = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+                const auto lo = __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf((float)hi[0], -1.0f, p0), __builtin_fmaf((float)hi[1], -1.0f, p1));
+                pb[j] = hi[0];
+                pb[j + 1] = hi[1];
+                pl[j] = lo[0];
+                pl[j + 1] = lo[1];
+            }
+            pf_half8 vf[4];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) vf[d] = *reinterpret_cast<const pf_half8*>(&bufs[buf][half].v[32 * d + tl][16 * u + 8 * h]);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[d], pb, o[d], 0, 0, 0);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[d], pl, o[d], 0, 0, 0);
+        }
+        // a step's probabilities are formed under the previous step's MFMAs
+        __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedValu, 40, 0);
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 4, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(kSchedValu, 5, 0);
+            }
+        }
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 8, 0);
+        if (round + 1 < rounds) stage_v(buf ^ 1, vp);
+        __syncthreads();
+    }
+
+    // ---- the second key half's state into the first's, through LDS
+    if constexpr (KS == 2) {
+        float4* const xo = reinterpret_cast<float4*>(lds) + wave * (17 * 64) + lane;
+        static_assert(W * 17 * 64 * (int)sizeof(float4) <= kLoop, "the half's state must fit");
+        if (half == 1) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                xo[64 * i] = make_float4(o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2],
+                                         o[i >> 2][4 * (i & 3) + 3]);
+            xo[64 * 16] = make_float4(m_run, l_run, 0.f, 0.f);
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const float4 ml = xo[64 * 16];
+        const float m_new = fmaxf(m_run, ml.x);
+        const float c0 = __builtin_amdgcn_exp2f(m_run - m_new), c1 = __builtin_amdgcn_exp2f(ml.x - m_new);
+        l_run = l_run * c0 + ml.y * c1;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float4 v = xo[64 * i];
+            const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[i >> 2][4 * (i & 3) + j] = o[i >> 2][4 * (i & 3) + j] * c0 + w[j] * c1;
+        }
+    }
+
+    // ---- the token's denominator over its two lanes, then O / l
+    const float l_tot = pair_combine(l_run, [](float u, float v) { return u + v; });
+    const float r_tot = 1.0f / l_tot;
+    if (!live) return;
+    float* dst = a.out + (size_t)t * qdim + (size_t)hq * kHeadDim + 4 * h;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>(dst + 32 * d + 8 * i) =
+                make_float4(o[d][4 * i] * r_tot, o[d][4 * i + 1] * r_tot, o[d][4 * i + 2] * r_tot, o[d][4 * i + 3] * r_tot);
+}
+
 }  // namespace
 
 size_t attn_partials_floats(int q_heads) { return (size_t)q_heads * kAttnChunks * kPartStride; }
@@ -974,6 +1389,32 @@ hipError_t launch_kv_append(const AttnArgs& args, int members, hipStream_t strea
     return hipGetLastError();
 }
 
+namespace {
+// Whether the wide form's grid fills enough of the 256 CUs (its workgroups take
+// one each, with a longer prologue). Measured, us, narrow / wide: 32 / 8 heads at
+// 512, 768, 1,024, 2,047 tokens (128, 192, 256, 512 workgroups) 27.0 / 29.2,
+// 41.5 / 37.2, 53.5 / 45.6, 139 / 96; 16 / 8 heads at 1,024, 1,400 (128, 176)
+// 40.6 / 42.0, 57.5 / 53.6; 8 / 8 heads at 1,024 (64) 45.4 / 41.0; 64 / 8 heads at
+// 512, 1,024 (128, 256) 31.0 / 42.9, 81.5 / 70.1.
+bool wide_prefill(const PrefillAttnArgs& a, int tiles) {
+    const int qpk = a.q_heads / a.kv_heads;
+    return tiles * a.kv_heads >= (qpk == 1 ? 64 : qpk == 8 ? 256 : 176);
+}
+
+template <int QPK>
+hipError_t launch_prefill_heads(const PrefillAttnArgs& a, hipStream_t stream) {
+    constexpr int TT = QPK < 4 ? 4 / QPK : 1;  // token tiles per workgroup
+    const int wide = (a.tokens + kPrefillWideTokens * TT - 1) / (kPrefillWideTokens * TT);
+    if (wide_prefill(a, wide)) {
+        hipLaunchKernelGGL(attn_prefill_wide_kernel<QPK>, dim3((unsigned)wide * (unsigned)a.kv_heads), dim3(512), 0, stream, a, wide);
+    } else {
+        const int tiles = (a.tokens + kPrefillTileTokens * TT - 1) / (kPrefillTileTokens * TT);
+        hipLaunchKernelGGL(attn_prefill_kernel<QPK>, dim3((unsigned)tiles, (unsigned)a.kv_heads), dim3(QPK < 8 ? 256 : 512), 0, stream, a);
+    }
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream) {
     if (a.tokens < 1 || a.kv_heads < 1 || a.q_heads % a.kv_heads != 0 || a.p0 < 0 ||
         (long long)a.p0 + a.tokens > a.mem.capacity || a.mem.keys == nullptr || a.mem.values == nullptr) {
@@ -982,17 +1423,13 @@ hipError_t launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream
     hipLaunchKernelGGL(kv_append_seq_kernel, dim3((unsigned)a.kv_heads, (unsigned)a.tokens), dim3(128), 0, stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.out == nullptr) return e;
-    const int qpk = a.q_heads / a.kv_heads;
-    const int tile = kPrefillTileTokens * (qpk < 4 ? 4 / qpk : 1);
-    const dim3 grid((unsigned)((a.tokens + tile - 1) / tile), (unsigned)a.kv_heads);
-    switch (qpk) {
-    case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(256), 0, stream, a); break;
-    case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(256), 0, stream, a); break;
-    case 4: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, dim3(256), 0, stream, a); break;
-    case 8: hipLaunchKernelGGL(attn_prefill_kernel<8>, grid, dim3(512), 0, stream, a); break;
+    switch (a.q_heads / a.kv_heads) {
+    case 1: return launch_prefill_heads<1>(a, stream);
+    case 2: return launch_prefill_heads<2>(a, stream);
+    case 4: return launch_prefill_heads<4>(a, stream);
+    case 8: return launch_prefill_heads<8>(a, stream);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_token_upload(const uint32_t* tokens, size_t count, uint32_t* dst, hipStream_t stream) {

@@ -123,8 +123,9 @@ struct PrefillAttnArgs {
     float scale;           // log2(e) / sqrt(head_dim)
 };
 
-// Tokens one prompt-attention workgroup tile covers per query head.
+// Tokens a prompt-attention wave covers (its wide form: many tokens).
 constexpr int kPrefillTileTokens = 16;
+constexpr int kPrefillWideTokens = 32;
 
 // The chunk's K (RMSNorm + rope) and V stored as f16 at their positions, then
 // (when `out` is set) causal attention of every token over positions

@@ -325,3 +325,46 @@ def test_prompt_errors(env):
     dec.prefill_prompt(cache, list(range(20)), 0, 16)  # still usable after the errors
     env["ctx"].synchronize()
     dec.close()
+
+
+@pytest.mark.parametrize("qh,kvh,p0,T", [(128, 128, 0, 33), (128, 128, 70, 129), (128, 64, 5, 139), (128, 32, 0, 163),
+                                         (128, 32, 61, 192), (128, 16, 3, 487), (32, 8, 0, 705), (32, 8, 1000, 768)])
+def test_wide_chunk_attention(env, qh, kvh, p0, T):
+    """The many-token form of the chunk attention (32 tokens a wave, two key halves): every GQA
+    width, ragged last tiles, chunks that continue a cache, against an f64 attention over the f16
+    keys and values the call left in the cache (the bound of the narrow form's test)."""
+    import torch
+    case(test="wide_chunk_attention", qh=qh, kvh=kvh, p0=p0, T=T)
+    E = env["E"]
+    cfg = dict(layers=1, hidden=4096, q_heads=qh, kv_heads=kvh, head_dim=128, ffn=256, vocab=1, rope_base=1.0e6,
+               epsilon=1.0e-6)
+    conf = E.AmdQwen3Config(**cfg)
+    cap = p0 + T + 3
+    rng = np.random.default_rng(qh + kvh + p0 + T)
+    cache = E.AmdKvCache(env["ctx"], conf, cap)
+    for ptr in cache.layer(0):
+        dev = rng.standard_normal((kvh, cap, 128)).astype(np.float16)
+        assert env["ctx"]._lib.ribn_amd_memcpy_htod(env["ctx"].handle, ctypes.c_void_p(ptr),
+                                                    dev.ctypes.data_as(ctypes.c_void_p), dev.nbytes) == 0
+    q = rng.standard_normal((T, qh * 128)).astype(np.float32)
+    k = rng.standard_normal((T, kvh * 128)).astype(np.float32)
+    v = (rng.standard_normal((T, kvh * 128)) * 4).astype(np.float32)
+    qn, kn = synth.gamma_numpy(128, 1), synth.gamma_numpy(128, 2)
+    out = to_dev(np.full(T * qh * 128, np.nan, np.float32))
+    E.attention_prefill(env["ctx"], conf, cache, 0, to_dev(q.reshape(-1)), to_dev(k.reshape(-1)), to_dev(v.reshape(-1)),
+                        to_dev(qn), to_dev(kn), T, p0, out)
+    got = to_host(out, env["ctx"]).reshape(T, qh, 128)
+    dev_k, dev_v = (torch.from_numpy(np.ascontiguousarray(a)).view(torch.float16).cuda().double()
+                    for a in cache_arrays(env, cache, cfg)[0])
+    qd = torch.from_numpy(q).cuda().double().view(T, qh, 128)
+    qd = qd * torch.rsqrt((qd * qd).mean(-1, keepdim=True) + 1e-6) * torch.from_numpy(qn).cuda().double()
+    pos = p0 + torch.arange(T, device="cuda:0")
+    ang = pos.double()[:, None] * 1.0e6 ** (-torch.arange(64, device="cuda:0").double() / 64)
+    cos, sin = ang.cos()[:, None], ang.sin()[:, None]
+    qd = torch.cat((qd[..., :64] * cos - qd[..., 64:] * sin, qd[..., :64] * sin + qd[..., 64:] * cos), -1)
+    seen = torch.arange(p0 + T, device="cuda:0")[None] <= pos[:, None]
+    for h in range(qh):
+        kh, vh = dev_k[h // (qh // kvh), :p0 + T], dev_v[h // (qh // kvh), :p0 + T]
+        sc = (qd[:, h] @ kh.t().contiguous()) / 128 ** 0.5
+        ref = (torch.softmax(sc.masked_fill(~seen, -np.inf), -1) @ vh).cpu().numpy()
+        assert max_rel_err(got[:, h], ref) <= ATTN_TOL, h

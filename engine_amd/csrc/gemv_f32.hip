@@ -255,7 +255,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
     constexpr int BB = BlockTraits<T>::bytes;
     constexpr int NBMAX = ONE_SLICE ? 16 : kF32Blocks;
     constexpr int NBW = (NBMAX + WAVES - 1) / WAVES;  // staging blocks per wave
-    extern __shared__ float xs[];                     // [MT][slices][64 records][STRIDE]
+    extern __shared__ __attribute__((aligned(16))) float xs[];                     // [MT][slices][64 records][STRIDE]
     __shared__ float ssq_s[NORM ? MT : 1][NORM ? NBMAX : 1];
 
     const int lane = threadIdx.x & 63;
@@ -576,6 +576,343 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
 
 namespace {
 
+// ---------------------------------------- one or two members, any super-blocks
+//
+// gemv_f32_slices_kernel: rows whose super-blocks are not one whole slice (K
+// above 4096, or at most 2048). A slice of 8 or fewer blocks leaves lanes idle
+// when a unit is one row, so a unit is RP = 1, 2 or 4 rows of a slice of up to
+// 16, 8 or 4 blocks (each row in 64 / RP lanes), and a wave keeps one slice's
+// records in VGPRs while it walks that slice's units: the workgroup's rows give
+// one sequence of units, slice by slice, cut evenly over its waves, so a wave
+// rereads records from LDS only where its share crosses a slice (before, at
+// every second row). Slice totals P_s meet in LDS; after one barrier a thread
+// per value adds them in slice order and applies the epilogue. The DPP row sums
+// of a unit's rows and the zeros an absent block would add make every row's
+// bits those of the one-slice form.
+//
+// Measured, one member, us (before: one row a unit, or pairs of rows over all
+// slices): Q4_K 5120 -> 17408 23.6 -> 16.3, Q6_K 29.7 -> 22.0; Q4_K 12288 ->
+// 17408 38.0 -> 32.0; 1024 -> 17408 8.9 -> 6.3; two members 5120 -> 17408 30.4 ->
+// 20.9. What bounds it: 3.1-4.0 TB/s of weights after a 4-6 us ramp; the
+// choice of form is launch_few's.
+constexpr int kSliceWaves = 8;
+
+// Rows of one slice a unit takes.
+__device__ __host__ constexpr int unit_rows(int blocks) { return blocks > 8 ? 1 : blocks > 4 ? 2 : 4; }
+
+template <int T, int MT, int PRO, bool MULTI, int NBUF, bool PAIR>
+__global__ __launch_bounds__(kSliceWaves * 64) void gemv_f32_slices_kernel(WaveGemvArgs args) {
+    static_assert(!PAIR || !MULTI, "pairs are one slice");
+    constexpr bool NORM = PRO == kProNorm;
+    constexpr bool SWIGLU = PRO == kProSwiglu;
+    constexpr int G = F32Rec<T>::groups;
+    constexpr int STRIDE = F32Rec<T>::stride;
+    constexpr int BB = BlockTraits<T>::bytes;
+    constexpr int WAVES = kSliceWaves;
+    constexpr int NBMAX = MULTI ? (MT == 1 ? 2 : 1) * kF32Blocks : 8;
+    constexpr int NBW = MULTI ? 6 : 1;                // blocks a wave stages at a time
+    extern __shared__ __attribute__((aligned(16))) float xs[];                     // [MT][slices][64 records][STRIDE], then the slice totals
+    __shared__ float ssq_s[NORM ? MT : 1][NORM ? NBMAX : 1];
+    __shared__ float inv_s[MT];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int K = args.K;
+    const int nb = K >> 8;
+    const int slices = MULTI ? (nb + 15) >> 4 : 1;
+    const int members = args.members;
+    const uint32_t row_bytes = (uint32_t)nb * BB;
+
+    // Rows in quads, numbered through the matrices (a matrix's last quad may be
+    // short); pairs: each quad of gate rows, then the up rows beside it.
+    int quad_end[kMaxGroup];
+#pragma unroll
+    for (int i = 0; i < kMaxGroup; ++i) {
+        const int rows = args.rows_end[i] - (i > 0 ? args.rows_end[i - 1] : 0);
+        quad_end[i] = (i > 0 ? quad_end[i - 1] : 0) + (i < args.count ? (rows + 3) >> 2 : 0);
+    }
+    const int quads_all = PAIR ? quad_end[0] : quad_end[kMaxGroup - 1];
+    const int q_begin = (int)((long long)quads_all * blockIdx.x / gridDim.x);
+    const int q_end = (int)((long long)quads_all * (blockIdx.x + 1) / gridDim.x);
+    const int quads = (PAIR ? 2 : 1) * (q_end - q_begin);  // of this workgroup
+    auto locate = [&](int quad, int& mat, int& row0) {
+        const int q = q_begin + (PAIR ? quad >> 1 : quad);
+        mat = 0;
+        int start = 0;
+        if constexpr (PAIR) {
+            mat = quad & 1;
+        } else {
+#pragma unroll
+            for (int i = 0; i < kMaxGroup - 1; ++i) {
+                if (i + 1 < args.count && q >= quad_end[i]) {
+                    mat = i + 1;
+                    start = quad_end[i];
+                }
+            }
+        }
+        row0 = 4 * (q - start);
+    };
+    // units of the last slice per quad, and the wave's share of the sequence
+    const int last_blocks = nb - 16 * (slices - 1);
+    const int last_rp = unit_rows(last_blocks);
+    const int full_units = 4 * quads * (slices - 1);
+    const int units = full_units + (4 / last_rp) * quads;
+    const int u_begin = (int)((long long)units * wave / WAVES);
+    const int u_end = (int)((long long)units * (wave + 1) / WAVES);
+
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(args.x, (uint32_t)members * (uint32_t)K * 4u);
+    const __amdgpu_buffer_rsrc_t gr = make_rsrc(args.gamma, NORM ? (uint32_t)K * 4u : 0u);
+    const __amdgpu_buffer_rsrc_t ur = make_rsrc(args.x2, SWIGLU ? (uint32_t)members * (uint32_t)K * 4u : 0u);
+
+    // A position in the unit sequence: the slice, the unit in it, and what that
+    // makes of this lane (its row of the unit, its record of the slice).
+    struct Place {
+        int slice, idx, end;  // unit of the slice, units the slice has
+        int rp;
+        uint32_t lane_off;    // of the lane's row and block from the unit's first row
+        bool live;            // the lane's block exists
+        int rec;
+    };
+    auto enter = [&](Place& c, int slice, int idx) {
+        c.slice = slice;
+        c.idx = idx;
+        c.rp = slice + 1 < slices ? 1 : last_rp;
+        c.end = (4 / c.rp) * quads;
+        const int lanes = 64 / c.rp;  // a power of two
+        c.rec = lane & (lanes - 1);
+        const int block = 16 * slice + (c.rec >> 2);
+        c.live = block < nb;
+        c.lane_off = (uint32_t)(lane / lanes) * row_bytes + (uint32_t)block * BB;
+    };
+    auto place = [&](int unit) {
+        Place c;
+        const int s = min(unit / (4 * quads > 0 ? 4 * quads : 1), slices - 1);
+        enter(c, s, unit - 4 * quads * s);
+        return c;
+    };
+    auto step = [&](Place& c) {
+        if (++c.idx == c.end) enter(c, min(c.slice + 1, slices - 1), 0);
+    };
+    const int p = lane & 3;
+    Place lp = place(u_begin);
+    RowData<T> ring[NBUF];
+    int lunit = u_begin;
+    auto load_next = [&](RowData<T>& dst) {
+        const int shift = lp.rp == 1 ? 2 : lp.rp == 2 ? 1 : 0;  // log2 units per quad
+        int mat, row0;
+        locate(lp.idx >> shift, mat, row0);
+        row0 += (lp.idx & ((1 << shift) - 1)) * lp.rp;
+        const uint8_t* w = args.w[0];
+        uint32_t bytes = args.wbytes[0];
+#pragma unroll
+        for (int i = 1; i < kMaxGroup; ++i) {
+            if (mat == i) {
+                w = args.w[i];
+                bytes = args.wbytes[i];
+            }
+        }
+        // dead units read through an empty resource; rows past the matrix lie
+        // past its bytes: zeros
+        load_row<T>(dst, make_rsrc(w, lunit < u_end ? bytes : 0u),
+                    lp.live ? lp.lane_off + (uint32_t)row0 * row_bytes : kOutOfRange, p);
+        ++lunit;
+        step(lp);
+    };
+
+    // ---- staging, as the one-slice form's, NBW blocks a wave at a time (all of
+    // K up to 12288; a longer unrolled run costs more in cold code): activation
+    // loads first, then, the first time, the first units of weights
+#pragma unroll 1
+    for (int b0 = wave; b0 < 16 * slices; b0 += WAVES * NBW) {
+        float4 xv[NBW][MT];
+        float4 gv[NORM ? NBW : 1];
+        float4 uv[SWIGLU ? NBW : 1][SWIGLU ? MT : 1];
+#pragma unroll
+        for (int k = 0; k < NBW; ++k) {
+            const int b = b0 + WAVES * k;
+            const int e = 256 * b + 4 * lane;
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                xv[k][m] = float4{0.f, 0.f, 0.f, 0.f};
+                if constexpr (SWIGLU) uv[k][m] = float4{0.f, 0.f, 0.f, 0.f};
+            }
+            if constexpr (NORM) gv[k] = float4{0.f, 0.f, 0.f, 0.f};
+            if (b < nb) {  // uniform: a wave issues only the loads its K has
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const uint32_t off = m < members ? (uint32_t)(m * K + e) * 4u : kOutOfRange;
+                    xv[k][m] = load_f4(xr, off);
+                    if constexpr (SWIGLU) uv[k][m] = load_f4(ur, off);
+                }
+                if constexpr (NORM) gv[k] = load_f4(gr, (uint32_t)e * 4u);
+            }
+        }
+        asm volatile("" ::: "memory");
+        if (b0 == wave) {
+#pragma unroll
+            for (int r = 0; r < NBUF; ++r) load_next(ring[r]);
+        }
+#pragma unroll
+        for (int k = 0; k < NBW; ++k) {
+            const int b = b0 + WAVES * k;
+            // blocks past K inside the last slice are staged as zeros
+            if (b >= 16 * slices) break;
+            const int slice = b >> 4;
+            int rec, pos;
+            f32_slot<T>(256 * (b & 15) + 4 * lane, rec, pos);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                float4 v = xv[k][m];
+                if constexpr (SWIGLU) {
+                    // silu(gate) * up, in the reference's operation order (model_ops.rs:316-328)
+                    v.x = (v.x / (1.0f + expf(-v.x))) * uv[k][m].x;
+                    v.y = (v.y / (1.0f + expf(-v.y))) * uv[k][m].y;
+                    v.z = (v.z / (1.0f + expf(-v.z))) * uv[k][m].z;
+                    v.w = (v.w / (1.0f + expf(-v.w))) * uv[k][m].w;
+                }
+                if constexpr (NORM) {
+                    const float sq = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+                    const float blk = wave_sum_uniform(sq);
+                    if (lane == 0 && b < nb && m < members) ssq_s[m][b] = blk;
+                    v.x *= gv[k].x;
+                    v.y *= gv[k].y;
+                    v.z *= gv[k].z;
+                    v.w *= gv[k].w;
+                }
+                const float gsum = group_sum_f<T>(((v.x + v.y) + v.z) + v.w);
+                float* dst = xs + ((m * slices + slice) * 64 + rec) * STRIDE;
+                *reinterpret_cast<float4*>(dst + pos) = v;
+                if ((lane & (F32Rec<T>::group / 4 - 1)) == 0) dst[64 + pos / F32Rec<T>::group] = gsum;
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < MT) {
+        float inv = 1.f;
+        if constexpr (NORM) {
+            if ((int)threadIdx.x < members) {
+                float total = 0.f;
+                for (int b = 0; b < nb; ++b) total += ssq_s[threadIdx.x][b];
+                // RMSNorm (qwen_reference.rs:550-556): x * (1/sqrt(sum(x^2)/K + eps)) * gamma
+                inv = 1.0f / sqrtf(total / (float)K + args.eps);
+            }
+        }
+        inv_s[threadIdx.x] = inv;
+    }
+
+    // slice totals: [row of the workgroup][slice][member]
+    float* const sums = xs + (size_t)MT * slices * 64 * STRIDE;
+    float4 xq[MT][16];
+    float xg[MT][G];
+    auto read_rec = [&](int slice, int rec) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const float* src = xs + ((m * slices + slice) * 64 + rec) * STRIDE;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) xq[m][i] = *reinterpret_cast<const float4*>(src + 4 * i);
+            const float4 s4 = *reinterpret_cast<const float4*>(src + 64);
+            const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+            for (int g = 0; g < G; ++g) xg[m][g] = sv[g];
+        }
+    };
+    auto xf = [&](int m, int i) { return xq[m][i]; };
+    auto sf = [&](int m, int g) { return xg[m][g]; };
+    Place cp = place(u_begin);
+    if (u_begin < u_end) read_rec(cp.slice, cp.rec);
+    auto consume = [&](const RowData<T>& d) {
+        float part[MT];
+        row_dot<T, MT>(d, p, xf, sf, part);
+        float* dst = sums + ((size_t)cp.idx * cp.rp * slices + cp.slice) * MT;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            float v = part[m];
+            v = dpp_step<0xb1>(v);   // quad_perm [1,0,3,2]
+            v = dpp_step<0x4e>(v);   // quad_perm [2,3,0,1]
+            v = dpp_step<0x141>(v);  // row_half_mirror
+            v = dpp_step<0x140>(v);  // row_mirror
+            const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
+            const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
+            const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
+            const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
+            // (+ 0: the sum an absent half or quarter of the slice would add)
+            if (cp.rp == 1) {
+                const float t = (r0 + r1) + (r2 + r3);
+                if (lane == 0) dst[m] = t;
+            } else if (cp.rp == 2) {
+                const float t = (lane == 0 ? r0 + r1 : r2 + r3) + 0.0f;
+                if (lane < 2) dst[lane * slices * MT + m] = t;
+            } else {
+                const float t = (lane == 0 ? r0 : lane == 1 ? r1 : lane == 2 ? r2 : r3) + 0.0f;
+                if (lane < 4) dst[lane * slices * MT + m] = t;
+            }
+        }
+        const int slice = cp.slice;
+        step(cp);
+        if (MULTI && cp.slice != slice) read_rec(cp.slice, cp.rec);
+    };
+    int left = u_end - u_begin;
+    for (; left > NBUF; left -= NBUF) {
+#pragma unroll
+        for (int r = 0; r < NBUF; ++r) {
+            consume(ring[r]);
+            load_next(ring[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < NBUF; ++r) {
+        if (r < left) consume(ring[r]);
+    }
+
+    // ---- rows: a value per thread, its address found before the barrier
+    const int rows_wg = 4 * (PAIR ? quads >> 1 : quads);
+    struct Out {
+        float* y;  // null: no value
+        int at, m;
+    };
+    auto out_of = [&](int v) {
+        Out o{nullptr, 0, MT == 1 ? 0 : v & 1};
+        const int r = MT == 1 ? v : v >> 1;
+        const int quad = PAIR ? 2 * (r >> 2) : r >> 2;
+        o.at = (4 * quad + (r & 3)) * slices * MT + o.m;
+        int mat, row0;
+        locate(quad, mat, row0);
+        const int rows = args.rows_end[mat] - (mat > 0 ? args.rows_end[mat - 1] : 0);
+        const int row = row0 + (r & 3);
+        if (r < rows_wg && row < rows && o.m < members) {
+            float* y = args.y[0];
+#pragma unroll
+            for (int i = 1; i < kMaxGroup; ++i)
+                if (!PAIR && mat == i) y = args.y[i];
+            o.y = y + (size_t)o.m * rows + row;
+        }
+        return o;
+    };
+    Out out = out_of(threadIdx.x);
+    __syncthreads();
+#pragma unroll 1
+    for (int v = threadIdx.x; v < rows_wg * MT; v += WAVES * 64) {
+        if (v >= WAVES * 64) out = out_of(v);
+        if (out.y == nullptr) continue;
+        auto total_at = [&](int at) {
+            float t = sums[at];
+            for (int s = 1; s < slices; ++s) t = t + sums[at + s * MT];
+            return t * inv_s[out.m];
+        };
+        float value = total_at(out.at);
+        if constexpr (PAIR) {
+            // silu(gate) * up (model_ops.rs:316-328); the up quad follows
+            const float up = total_at(out.at + 4 * slices * MT);
+            value = (value / (1.0f + expf(-value))) * up;
+        }
+        if (args.accumulate) {
+            unsafeAtomicAdd(out.y, value);
+        } else {
+            *out.y = value;
+        }
+    }
+}
+
 // ------------------------------------------- three to eight members, MFMA
 //
 // gemv_f32_many_kernel: the same rows for 3..8 members, one slice per
@@ -740,7 +1077,7 @@ __global__ __launch_bounds__(kManyWaves * 64) void gemv_f32_many_kernel(WaveGemv
     constexpr int MT = 4 * MG;
     constexpr int BB = BlockTraits<T>::bytes;
     constexpr int NBW = 16 / kManyWaves;  // staging blocks per wave
-    extern __shared__ float xs[];         // [MT][64 records][68] (member stride kManyStride), then the units' block sums
+    extern __shared__ __attribute__((aligned(16))) float xs[];         // [MT][64 records][68] (member stride kManyStride), then the units' block sums
     __shared__ float ssq_s[NORM && !SPLIT ? MT : 1][NORM && !SPLIT ? 16 : 1];
     __shared__ float inv_s[MT];
 
@@ -1064,15 +1401,60 @@ __global__ __launch_bounds__(256) void f32_split_reduce_kernel(WaveGemvArgs a, i
     }
 }
 
+// One or two members whose K is not one slice of more than 8 blocks.
+template <int T, int MT, int PRO, bool MULTI, bool PAIR = false>
+hipError_t launch_slices(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
+    constexpr int kRing = 2;
+    constexpr int kMaxLds = 158 * 1024;  // beside the kernel's own few hundred bytes
+    auto kern = gemv_f32_slices_kernel<T, MT, PRO, MULTI, kRing, PAIR>;
+    static std::atomic<bool> sized{false};
+    if (!sized.load(std::memory_order_relaxed)) {
+        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+        if (e != hipSuccess) return e;
+        sized.store(true, std::memory_order_relaxed);
+    }
+    const int nb = a.K >> 8, slices = (nb + 15) >> 4;
+    long long quads = 0;
+    for (int i = 0; i < (PAIR ? 1 : a.count); ++i)
+        quads += (a.rows_end[i] - (i > 0 ? a.rows_end[i - 1] : 0) + 3) / 4;
+    // one workgroup per CU, fewer where a wave would have less than a unit or
+    // two, more where a workgroup's slice totals would not fit beside its records
+    const long long records = (long long)MT * slices * 64 * F32Rec<T>::stride * 4;
+    const long long quad_bytes = (PAIR ? 2LL : 1LL) * 4 * slices * MT * 4;
+    const long long quad_units = (PAIR ? 2 : 1) * (4LL * (slices - 1) + 4 / unit_rows(nb - 16 * (slices - 1)));
+    long long grid = std::min<long long>(cu_count, (quads * quad_units + kSliceWaves - 1) / kSliceWaves);
+    const long long most = (kMaxLds - records) / quad_bytes;  // quads a workgroup holds
+    if (most < 1) return hipErrorInvalidValue;
+    grid = std::max<long long>({grid, 1, (quads + most - 1) / most});
+    grid = std::min(grid, quads);
+    const long long held = (quads + grid - 1) / grid;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kSliceWaves * 64), (size_t)(records + held * quad_bytes), stream, a);
+    return hipGetLastError();
+}
+
 // One or two members.
 template <int T, int MT, int PRO, bool ONE_SLICE, bool PAIR = false>
 hipError_t launch_few(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
-    const int slices = ONE_SLICE ? 1 : ((a.K >> 8) + 15) >> 4;
-    const long long units = (long long)a.total_rows * slices;
-    const long long per_cu = (units + cu_count - 1) / cu_count;
     if constexpr (!ONE_SLICE) {
-        return F32Instance<T, MT, PRO, false, 2, 8, 2>::launch(a, cu_count, 1, stream);
+        // One pair of rows per wave over (nearly) every wave is where reading
+        // the records once a pair costs least: up to 16 rows per CU that form
+        // stays (Q4_K, one member, us, pairs / slices: K 5120 at 3072, 4096,
+        // 5120 rows 6.9 / 6.3, 7.1 / 7.7, 10.7 / 8.4; K 12288 at 2048, 3072, 4096,
+        // 5120 rows 8.9 / 8.2, 9.6 / 10.2, 10.2 / 11.2, 15.7 / 13.1).
+        const long long from = (a.K <= 2 * kSliceElems ? 15LL : 11LL) * cu_count;
+        if (a.total_rows > from && a.total_rows <= 16LL * cu_count) {
+            return F32Instance<T, MT, PRO, false, 2, 8, 2>::launch(a, cu_count, 1, stream);
+        }
+        return launch_slices<T, MT, PRO, true>(a, cu_count, stream);
     } else {
+        // Short rows: several to a unit, where the launch is long enough for it
+        // (Q4_K, one member, us, one row / several: K 1024 at 4096, 5120, 12288
+        // rows 4.2 / 4.6, 5.0 / 4.7, 7.0 / 5.7; K 2048 at 8192, 12288, 17408 rows
+        // 5.6 / 5.9, 7.8 / 7.5, 9.8 / 8.7).
+        if (a.total_rows > (a.K <= 1024 ? 16LL : 40LL) * cu_count && a.K <= 2048) {
+            return launch_slices<T, MT, PRO, false, PAIR>(a, cu_count, stream);
+        }
+        const long long per_cu = ((long long)a.total_rows + cu_count - 1) / cu_count;
         if constexpr (MT == 1) {
             // Streams of more than 48 units per CU (gate/up, the lm_head): a
             // three-unit ring (four for gate/up pairs) over 8-wave workgroups,
@@ -1171,6 +1553,7 @@ hipError_t launch_type(const WaveGemvArgs& a, int cu_count, hipStream_t stream) 
 // its records in VGPRs, as the one-launch form does.
 template <int T>
 hipError_t launch_split(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
+    if (a.members == 1 && a.K <= 2 * kWaveMaxK) return launch_slices<T, 1, kProPlain, true>(a, cu_count, stream);
     hipError_t e = (a.members == 1)
                        ? F32Instance<T, 1, kProPlain, true, 3, 8, 1, false, true>::launch(a, cu_count, 1, stream)
                    : a.gamma != nullptr ? launch_many<T, kProNorm, false, true>(a, cu_count, stream)

@@ -717,3 +717,71 @@ def test_many_members_edges_bit_identical(env, t, blocks, ns, members, norm):
     kern.execute_fused(ws[0], to_dev(x.reshape(-1)), acc, members, gamma=g, epsilon=1e-6, accumulate=True)
     want = base + to_host(ys[0], env["ctx"])
     assert np.array_equal(to_host(acc, env["ctx"]).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("t,blocks,ns,pro", [
+    (12, 1, (4099, 30), "norm"), (13, 2, (4500,), ""), (14, 3, (4097, 3), ""), (12, 4, (6001,), "norm"),
+    (14, 5, (10300,), ""), (13, 8, (10245, 6), "norm"), (12, 17, (131, 4), ""), (13, 20, (4133,), "norm"),
+    (14, 24, (77, 1000), ""), (12, 33, (5001,), "swiglu"), (13, 48, (4100,), ""), (14, 64, (515,), "norm"),
+    (12, 68, (321,), ""), (13, 128, (37,), "")])
+def test_slices_form_edges(env, t, blocks, ns, pro):
+    """One and two members over rows that are not one whole slice: several short rows to a unit (1..8
+    super-blocks) and waves that keep one slice (17..128), with ragged last quads in each matrix, every
+    prologue and the accumulating form: rows of one member against the oracle at the f32 bar, two
+    members bit-identical to it, and three (the matrix-core form) too."""
+    k = 256 * blocks
+    print_case(test="slices_edges", t=t, k=k, ns=ns, pro=pro)
+    encs = [synth.kquant_numpy(t, k, n, seed=k + n + j) for j, n in enumerate(ns)]
+    ws = [upload(env, t, k, n, e) for n, e in zip(ns, encs)]
+    x = synth.activations_numpy(k, 3, seed=17 * blocks)
+    gamma = synth.gamma_numpy(k, seed=blocks)
+    up = synth.activations_numpy(k, 3, seed=5)
+    kern = env["k"][t]
+
+    def run(m):
+        ys = [empty_dev(m * n) for n in ns]
+        xin = to_dev(x[:m].reshape(-1))
+        if pro == "swiglu":
+            kern.execute_fused(ws[0], xin, ys[0], m, up=to_dev(up[:m].reshape(-1)))
+        else:
+            kern.execute_group(ws, xin, ys, m, gamma=to_dev(gamma) if pro == "norm" else None, epsilon=1e-6)
+        return [to_host(y, env["ctx"]).reshape(m, n) for y, n in zip(ys, ns)]
+
+    one, two = run(1), run(2)
+    three = run(3) if pro != "swiglu" and (pro == "" or k <= 16384) else None
+    xin = {"norm": lambda: O.rms_norm_raw(x[0], gamma, 1e-6), "swiglu": lambda: O.swiglu(x[0], up[0]), "": lambda: x[0]}[pro]()
+    for j, n in enumerate(ns):
+        assert max_rel_err(one[j][0], O.quant_gemv(t, encs[j], k, n, xin, threads=8)) <= F32_RTOL
+        for other in (two, three):
+            if other is not None:
+                assert np.array_equal(other[j][0].view(np.uint32), one[j][0].view(np.uint32))
+    if pro == "":
+        base = synth.activations_numpy(ns[0], 1, seed=3).reshape(-1)
+        acc = to_dev(base)
+        kern.execute_fused(ws[0], to_dev(x[0]), acc, 1, accumulate=True)
+        assert np.array_equal(to_host(acc, env["ctx"]).view(np.uint32), (base + one[0][0]).view(np.uint32))
+
+
+@pytest.mark.parametrize("t,blocks,n", [(12, 4, 2057), (13, 7, 5130), (14, 8, 5121)])
+def test_slices_form_gate_up_pairs(env, t, blocks, n):
+    """Gate/up pairs of short rows (several to a unit): one member's silu(gate) * up bit-identical to
+    the pair formed from the separate products, two and three members to one."""
+    k = 256 * blocks
+    print_case(test="slices_pairs", t=t, k=k, n=n)
+    ws = [upload(env, t, k, n, synth.kquant_numpy(t, k, n, seed=k + n + j)) for j in range(2)]
+    x = synth.activations_numpy(k, 3, seed=n) * np.float32(0.02)
+    gamma = to_dev(synth.gamma_numpy(k, seed=blocks))
+    kern = env["k"][t]
+    outs = []
+    for m in (1, 2, 3):
+        y = empty_dev(m * n)
+        kern.execute_gate_up_swiglu(ws[0], ws[1], to_dev(x[:m].reshape(-1)), y, m, gamma=gamma, epsilon=1e-6)
+        outs.append(to_host(y, env["ctx"]).reshape(m, n))
+    assert np.array_equal(outs[1][0].view(np.uint32), outs[0][0].view(np.uint32))
+    assert np.array_equal(outs[2][:2].view(np.uint32), outs[1].view(np.uint32))
+    parts = []
+    for w in ws:
+        y = empty_dev(n)
+        kern.execute_rms_norm(w, to_dev(x[0]), gamma, 1e-6, y, 1)
+        parts.append(to_host(y, env["ctx"]))
+    assert max_rel_err(outs[0][0], O.swiglu(parts[0], parts[1])) <= 1e-6  # expf's last bits

@@ -428,8 +428,14 @@ __device__ __forceinline__ void lds_done_barrier() { asm volatile("s_waitcnt lgk
 // ever waits on a load at a barrier: block b's fragments are complete when
 // the loader reaches barrier b, and the compute waves' weight loads run NS - 1
 // blocks ahead, independent of the barriers.
-template <int T, int R, int MT, bool PAIR, int NL, int NS>
+//
+// MS = 2 (pairs of two or four member tiles): two waves share a unit of R row
+// tiles, half of the member tiles each: the weights are dequantised twice, in
+// time that SIMDs without a wave had (launch_shape).
+template <int T, int R, int MT, bool PAIR, int NL, int NS, int MS>
 __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
+    static_assert(MT % MS == 0, "whole member tiles per wave");
+    constexpr int MTW = MT / MS;  // member tiles of a compute wave
     constexpr int BB = BlockTraits<T>::bytes;
     constexpr int PC = pieces_of<T>();
     constexpr int FRAGS = MT * 8 * PC;  // 1 KB fragment loads per block
@@ -476,7 +482,8 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int W = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6)) - 1;  // compute waves
+    const int waves = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6)) - 1;  // compute waves
+    const int W = waves / MS;                                                      // units of R row tiles
     const int kq = lane >> 4, rl = lane & 15;
     const int nb = A.K >> 8;
     const uint32_t row_bytes = (uint32_t)nb * BB;
@@ -484,7 +491,7 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
     const int sb1 = min(nb, sb0 + A.split_blocks);
     const int tile0 = A.member0 >> 4;
 
-    if (wave == W) {
+    if (wave == waves) {
         // ---- loader: block b's fragments into LDS slot (b - sb0) % NL; past
         // the range the loads read zeros into a slot nobody reads
         const __amdgpu_buffer_rsrc_t ar = make_rsrc(A.act, A.act_bytes);
@@ -541,7 +548,10 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
         return;
     }
 
-    // this wave's tiles: (matrix, first local row); tiles never straddle matrices
+    // this wave's tiles: (matrix, first local row); tiles never straddle
+    // matrices; and the first of its member tiles
+    const int unit = wave / MS;
+    const int mt0 = (wave % MS) * MTW;
     __amdgpu_buffer_rsrc_t wr[R];
     int mat[R], local0[R], rows_mat[R], vrow0[R];
     bool live_row[R];
@@ -550,11 +560,11 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
     for (int i = 0; i < R; ++i) {
         if constexpr (PAIR) {
             mat[i] = i / (R / 2);
-            local0[i] = (((int)blockIdx.x * W + wave) * (R / 2) + i % (R / 2)) * 16;
+            local0[i] = (((int)blockIdx.x * W + unit) * (R / 2) + i % (R / 2)) * 16;
             rows_mat[i] = A.rows_end[0];
             vrow0[i] = (mat[i] ? A.rows_end[0] : 0) + local0[i];
         } else {
-            const int row0 = (((int)blockIdx.x * W + wave) * R + i) * 16;
+            const int row0 = (((int)blockIdx.x * W + unit) * R + i) * 16;
             int mm = 0, start = 0;
 #pragma unroll
             for (int j = 0; j < kMaxGroup - 1; ++j) {
@@ -584,11 +594,11 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
         rowoff[i] = live_row[i] ? (uint32_t)lrow * row_bytes : 0u;
     }
 
-    v4f acc[R][MT], macc[R][MT];
+    v4f acc[R][MTW], macc[R][MTW];
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
+        for (int mt = 0; mt < MTW; ++mt) {
             acc[i][mt] = (v4f){0.f, 0.f, 0.f, 0.f};
             macc[i][mt] = (v4f){0.f, 0.f, 0.f, 0.f};
         }
@@ -628,8 +638,8 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
             // minimum term of groups kq and 4 + kq (the lane's k slot):
             // A = X [member][group], B = dmin m [group][row]
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const float2 xs = xa[mt * 64 + lane];
+            for (int mt = 0; mt < MTW; ++mt) {
+                const float2 xs = xa[(mt0 + mt) * 64 + lane];
 #pragma unroll
                 for (int i = 0; i < R; ++i) {
                     macc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs.x, bmin0[i], macc[i][mt], 0, 0, 0);
@@ -644,7 +654,7 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
             // mixes four scale groups, every element carrying its own scale
             // (the packed activations follow the same order).
             const v4f zero = {0.f, 0.f, 0.f, 0.f};
-            v4f ch[R][MT], cl[R][MT];
+            v4f ch[R][MTW], cl[R][MTW];
             h2v sc2[R][4], nsc2[R][4];
 #pragma unroll
             for (int i = 0; i < R; ++i) {
@@ -678,8 +688,8 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
                     bq[i] = f16_scaled_quants(q0, q1, sc2[i][2 * L + hn], nsc2[i][2 * L + hn]);
                 }
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int f = (mt * 8 + c) * PC;
+                for (int mt = 0; mt < MTW; ++mt) {
+                    const int f = ((mt0 + mt) * 8 + c) * PC;
                     const v8h a0 = __builtin_bit_cast(v8h, fa[(f + 0) * 64 + lane]);
                     const v8h a1 = __builtin_bit_cast(v8h, fa[(f + 1) * 64 + lane]);
 #pragma unroll
@@ -692,8 +702,8 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
             }
             const float* const isa = isa_of(slot_c);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const float4 inv4 = *reinterpret_cast<const float4*>(isa + mt * 64 + 4 * kq);
+            for (int mt = 0; mt < MTW; ++mt) {
+                const float4 inv4 = *reinterpret_cast<const float4*>(isa + (mt0 + mt) * 64 + 4 * kq);
                 const float inv[4] = {inv4.x, inv4.y, inv4.z, inv4.w};
 #pragma unroll
                 for (int i = 0; i < R; ++i)
@@ -715,8 +725,8 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
                     bq1[i] = bf16_of_sbytes(low ? 0u : q0, low ? 0u : q1);
                 }
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    const int f = (mt * 8 + g) * PC;
+                for (int mt = 0; mt < MTW; ++mt) {
+                    const int f = ((mt0 + mt) * 8 + g) * PC;
                     const v8bf a0 = __builtin_bit_cast(v8bf, fa[(f + 0) * 64 + lane]);
                     const v8bf a1 = __builtin_bit_cast(v8bf, fa[(f + 1) * 64 + lane]);
                     const v8bf a2 = __builtin_bit_cast(v8bf, fa[(f + 2) * 64 + lane]);
@@ -765,11 +775,11 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
     StaticFor<0, NS - 1>::run(tail);
 
     // ---- epilogue: each wave owns its rows over the whole range
-    float v[R][MT][4];
+    float v[R][MTW][4];
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
             for (int t = 0; t < 4; ++t) v[i][mt][t] = acc[i][mt][t] - macc[i][mt][t];
     if (A.splits > 1) {
@@ -781,10 +791,10 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
 #pragma unroll
         for (int i = 0; i < R; ++i)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+            for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const int ml = 16 * mt + 4 * kq + t;  // member within the launch
+                    const int ml = 16 * (mt0 + mt) + 4 * kq + t;  // member within the launch
                     const bool ok = live_row[i] && ml < A.count_here;
                     const uint32_t off =
                         ok ? (uint32_t)(((int)blockIdx.y * A.count_here + ml) * vrows + vrow0[i] + rl) * 4u : kOOR;
@@ -792,13 +802,13 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
                 }
         return;
     }
-    float inv[MT][4];
+    float inv[MTW][4];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             inv[mt][t] = 1.f;
-            const int mem = A.member0 + 16 * mt + 4 * kq + t;
+            const int mem = A.member0 + 16 * (mt0 + mt) + 4 * kq + t;
             if (A.has_norm && mem < A.members) {
                 const float* ssq = reinterpret_cast<const float*>(A.act + A.L.ssq);
                 const float total = sum_in_order(ssq + mem * A.L.parts, A.L.parts);
@@ -820,15 +830,15 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
 #pragma unroll
         for (int i = 0; i < R / 2; ++i)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+            for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const int mem = A.member0 + 16 * mt + 4 * kq + t;
+                    const int mem = A.member0 + 16 * (mt0 + mt) + 4 * kq + t;
                     const float gt = v[i][mt][t] * inv[mt][t];
                     const float up = v[i + R / 2][mt][t] * inv[mt][t];
                     // silu(gate) * up, in the reference's operation order (model_ops.rs:316-328)
                     const float out = (gt / (1.0f + expf(-gt))) * up;
-                    const bool ok = live_row[i] && mem < A.members && 16 * mt + 4 * kq + t < A.count_here;
+                    const bool ok = live_row[i] && mem < A.members && 16 * (mt0 + mt) + 4 * kq + t < A.count_here;
                     put(out, yr, ok ? (uint32_t)(mem * ffn + local0[i] + rl) * 4u : kOOR);
                 }
     } else {
@@ -842,11 +852,11 @@ __global__ __launch_bounds__(512) void f32mma_gemv_kernel(F32MmaArgs A) {
             }
             const __amdgpu_buffer_rsrc_t yr = make_rsrc(y, (uint32_t)A.members * (uint32_t)rows_mat[i] * 4u);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+            for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const int mem = A.member0 + 16 * mt + 4 * kq + t;
-                    const bool ok = live_row[i] && mem < A.members && 16 * mt + 4 * kq + t < A.count_here;
+                    const int mem = A.member0 + 16 * (mt0 + mt) + 4 * kq + t;
+                    const bool ok = live_row[i] && mem < A.members && 16 * (mt0 + mt) + 4 * kq + t < A.count_here;
                     put(v[i][mt][t] * inv[mt][t], yr, ok ? (uint32_t)(mem * rows_mat[i] + local0[i] + rl) * 4u : kOOR);
                 }
         }
@@ -985,8 +995,25 @@ template <int T, int R, int MT, bool PAIR>
 hipError_t launch_shape(F32MmaArgs a, const F32MmaShape& sh, hipStream_t stream) {
     a.splits = sh.splits;
     a.split_blocks = sh.split_blocks;
-    hipLaunchKernelGGL((f32mma_gemv_kernel<T, R, MT, PAIR, lds_slots<T, MT>(), ring_depth<T, R, MT>()>),
-                       dim3((unsigned)sh.groups, (unsigned)sh.splits), dim3(64 * (sh.waves + 1)), 0, stream, a);
+    const dim3 grid((unsigned)sh.groups, (unsigned)sh.splits);
+    bool launched = false;
+    if constexpr (PAIR && MT % 2 == 0) {
+        // Where a workgroup holds one unit, and for Q4_K at four member tiles.
+        // Measured, gate/up at 24 / 64 members, us, one wave a unit / two:
+        // 4096 -> 2 x 4096 (one unit) Q4_K 21.9 / 20.7 and 31.0 / 26.9, Q6_K
+        // 42.9 / 40.4 and 82.5 / 77.7; 4096 -> 2 x 12288 (three) Q4_K 32.7 / 37.0
+        // and 48.4 / 46.7, Q5_K 38.2 / 45.4 and 54.2 / 55.7. (Single products
+        // were slower with two at every shape tried.)
+        if (sh.waves == 1 || (T == kQ4K && MT == 4 && 2 * sh.waves + 1 <= 8)) {
+            hipLaunchKernelGGL((f32mma_gemv_kernel<T, R, MT, PAIR, lds_slots<T, MT>(), ring_depth<T, R, MT>(), 2>), grid,
+                               dim3(64 * (2 * sh.waves + 1)), 0, stream, a);
+            launched = true;
+        }
+    }
+    if (!launched) {
+        hipLaunchKernelGGL((f32mma_gemv_kernel<T, R, MT, PAIR, lds_slots<T, MT>(), ring_depth<T, R, MT>(), 1>), grid,
+                           dim3(64 * (sh.waves + 1)), 0, stream, a);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.splits == 1 || a.skip_reduce) return e;
     const int rows = a.pair_swiglu ? a.rows_end[0] : a.total_rows;

@@ -231,3 +231,27 @@ def test_config2_ffn_shapes(env, members):
         assert np.all(np.isfinite(got[nm]))
         for m in sample:
             assert max_rel_err(got[nm][m], O.quant_gemv(t, e, k, n, src[m], threads=16)) <= F32_RTOL, (nm, m)
+
+
+@pytest.mark.parametrize("t,k,n,members", [(12, 512, 48, 24), (13, 768, 272, 64), (14, 512, 304, 33), (12, 1024, 4096, 50),
+                                           (12, 512, 12304, 61)])
+def test_gate_up_pair_two_waves_a_unit(env, t, k, n, members):
+    """Gate/up pairs whose member tiles two waves share (one unit a workgroup; Q4_K at four tiles):
+    silu(gate) * up of the separate products (the same chains per member, summed alike up to their
+    split), and members bit-identical to a 9-member call."""
+    case(test="pair_two_waves", t=t, k=k, n=n, members=members)
+    ws = [upload(env, t, k, n, synth.kquant_numpy(t, k, n, seed=k + n + j)) for j in range(2)]
+    x = synth.activations_numpy(k, members, seed=n) * np.float32(0.02)
+    kern = env["k"][t]
+    y = empty_dev(members * n)
+    kern.execute_gate_up_swiglu(ws[0], ws[1], to_dev(x.reshape(-1)), y, members)
+    got = to_host(y, env["ctx"]).reshape(members, n)
+    parts = []
+    for w in ws:
+        y = empty_dev(members * n)
+        kern.execute_warp_batch(w, to_dev(x.reshape(-1)), y, members)
+        parts.append(to_host(y, env["ctx"]))
+    assert max_rel_err(got.reshape(-1), O.swiglu(parts[0], parts[1])) <= F32_RTOL
+    y = empty_dev(9 * n)
+    kern.execute_gate_up_swiglu(ws[0], ws[1], to_dev(x[members - 9:].reshape(-1)), y, 9)
+    assert np.array_equal(to_host(y, env["ctx"]).reshape(9, n).view(np.uint32), got[members - 9:].view(np.uint32))

@@ -232,6 +232,14 @@ hipError_t launch_act_f16(bool bf16_in, const void* x, const float* gamma, float
                           hipStream_t stream);
 hipError_t launch_qgemm(int value_type, const uint8_t* w, uint32_t wbytes, void* workspace, size_t workspace_bytes,
                         float* y, int M, int N, int K, int cu_count, hipStream_t stream);
+// Two matrices of one type and shape over the same activations (k and v of a
+// prompt chunk): one launch of 256-row tiles with K split where the pair fills
+// the CUs together and neither does alone, else two launches. Measured, Q4_K
+// 4096 -> 1024 twice, reductions included: 300 tokens 56 -> 24 us, 2,047 tokens
+// 87 -> 60 us.
+hipError_t launch_qgemm_pair(int value_type, const uint8_t* w0, const uint8_t* w1, uint32_t wbytes, void* workspace,
+                             size_t workspace_bytes, float* y0, float* y1, int M, int N, int K, int cu_count,
+                             hipStream_t stream);
 // Activation stages of the decoder's prompt prefill (f32 [M][K], K a multiple
 // of 8): x += r (stored back to x), then RMSNorm with gamma, into the f16
 // workspace; or silu(gate) * up into it.

@@ -523,9 +523,13 @@ constexpr int kMaxReduceSplits = 16;
 template <int V>
 __global__ __launch_bounds__(256) void qgemm_reduce_kernel(const float* __restrict__ partial,
                                                            const float* __restrict__ unscale, float* __restrict__ y,
-                                                           int M, int N, int splits) {
+                                                           float* __restrict__ y2, int M, int N, int splits) {
     typedef float vec_t __attribute__((ext_vector_type(V)));
     const size_t total = (size_t)M * N;
+    if (blockIdx.y != 0) {  // the second matrix of a pair
+        partial += (size_t)splits * total;
+        y = y2;
+    }
     const size_t units = total / V;
     const size_t per_row = (size_t)N / V;
     const vec_t* __restrict__ pv = reinterpret_cast<const vec_t*>(partial);
@@ -543,16 +547,17 @@ __global__ __launch_bounds__(256) void qgemm_reduce_kernel(const float* __restri
     }
 }
 
-static hipError_t launch_reduce(const float* part, const float* us, float* y, int M, int N, int splits, int cu_count,
-                                hipStream_t stream) {
+static hipError_t launch_reduce(const float* part, const float* us, float* y, float* y2, int M, int N, int splits,
+                                int cu_count, hipStream_t stream) {
     if (splits < 2 || splits > kMaxReduceSplits) return hipErrorInvalidValue;
-    const bool wide = N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+    const bool wide = N % 4 == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(y2)) & 15u) == 0;
+    const unsigned mats = y2 != nullptr ? 2 : 1;
     const size_t units = (size_t)M * N / (wide ? 4 : 1);
     const int rgrid = (int)std::min<size_t>((units + 255) / 256, (size_t)std::max(1, cu_count) * 8);
     if (wide)
-        hipLaunchKernelGGL(qgemm_reduce_kernel<4>, dim3(rgrid), dim3(256), 0, stream, part, us, y, M, N, splits);
+        hipLaunchKernelGGL(qgemm_reduce_kernel<4>, dim3(rgrid, mats), dim3(256), 0, stream, part, us, y, y2, M, N, splits);
     else
-        hipLaunchKernelGGL(qgemm_reduce_kernel<1>, dim3(rgrid), dim3(256), 0, stream, part, us, y, M, N, splits);
+        hipLaunchKernelGGL(qgemm_reduce_kernel<1>, dim3(rgrid, mats), dim3(256), 0, stream, part, us, y, y2, M, N, splits);
     return hipGetLastError();
 }
 
@@ -725,7 +730,8 @@ __device__ __forceinline__ int tile_k0(int q) {
 template <int T, int RB, int TB>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void qgemm_tile_kernel(
     const uint8_t* __restrict__ w, uint32_t wbytes, const _Float16* __restrict__ xh, const float* __restrict__ unscale,
-    float* __restrict__ y, float* __restrict__ partial, int M, int N, int K, int split_sb) {
+    float* __restrict__ y, float* __restrict__ partial, int M, int N, int K, int split_sb,
+    const uint8_t* __restrict__ w2, float* __restrict__ y2, int tiles1) {
     constexpr int kTok = 16 * TB;                        // tokens per workgroup
     constexpr int kWaveTok = kTok / (kTileThreads / 64);  // x tile tokens each wave loads
     constexpr int kLoads = kWaveTok / 2;                  // its 1 KB loads per super-block
@@ -739,7 +745,13 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(1,
     const int wave = threadIdx.x >> 6;
     const int q = lane >> 4;
     const int r16 = lane & 15;
-    const int n0 = blockIdx.x * 64 * RB + 16 * RB * wave;
+    // row tiles from tiles1 on are the second matrix's (of the same shape)
+    const bool second = (int)blockIdx.x >= tiles1;
+    if (second) {
+        w = w2;
+        y = y2;
+    }
+    const int n0 = ((int)blockIdx.x - (second ? tiles1 : 0)) * 64 * RB + 16 * RB * wave;
     const int m0 = blockIdx.y * kTok;
     const int nb = K >> 8;
     const int sb_begin = blockIdx.z * split_sb;
@@ -896,7 +908,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(1,
     if (sb < sb_end) step(I0{}, std::false_type{}, sb);
 
     // epilogue: C[n][m] -> y[m][n] * unscale[m], or the raw split tile
-    float* out = partial ? partial + (size_t)blockIdx.z * M * N : y;
+    float* out = partial ? partial + ((size_t)blockIdx.z + (second ? gridDim.z : 0u)) * M * N : y;
     const bool vec = (N & 3) == 0;
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
@@ -996,7 +1008,7 @@ static hipError_t launch_qgemm_t(const uint8_t* w, uint32_t wbytes, void* worksp
                        splits > 1 ? part : nullptr, M, N, K, split_steps);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
-    return launch_reduce(part, us, y, M, N, splits, cu_count, stream);
+    return launch_reduce(part, us, y, nullptr, M, N, splits, cu_count, stream);
 }
 
 // Wide tiles. M > 128 runs 192-row x 128-token workgroups when their grid
@@ -1069,7 +1081,8 @@ static TileChoice choose_tile_small(int M, int N, int K, size_t room_bytes, int 
 
 template <int T, int RB, int TB>
 static hipError_t launch_tile_t(void* workspace, const uint8_t* w, uint32_t wbytes, float* y, int M, int N, int K,
-                                int splits, int cu_count, hipStream_t stream) {
+                                int splits, int cu_count, hipStream_t stream, const uint8_t* w2 = nullptr,
+                                float* y2 = nullptr) {
     uint8_t* base = static_cast<uint8_t*>(workspace);
     const _Float16* xh = reinterpret_cast<const _Float16*>(base);
     const size_t us_off = align256((size_t)M * K * 2);
@@ -1078,12 +1091,13 @@ static hipError_t launch_tile_t(void* workspace, const uint8_t* w, uint32_t wbyt
     const int nb = K >> 8;
     const int split_sb = (nb + splits - 1) / splits;
     splits = (nb + split_sb - 1) / split_sb;
-    const dim3 grid((N + 64 * RB - 1) / (64 * RB), (M + 16 * TB - 1) / (16 * TB), splits);
+    const int tiles1 = (N + 64 * RB - 1) / (64 * RB);
+    const dim3 grid(w2 != nullptr ? 2 * tiles1 : tiles1, (M + 16 * TB - 1) / (16 * TB), splits);
     hipLaunchKernelGGL((qgemm_tile_kernel<T, RB, TB>), grid, dim3(kTileThreads), 0, stream, w, wbytes, xh, us, y,
-                       splits > 1 ? part : nullptr, M, N, K, split_sb);
+                       splits > 1 ? part : nullptr, M, N, K, split_sb, w2, y2, tiles1);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
-    return launch_reduce(part, us, y, M, N, splits, cu_count, stream);
+    return launch_reduce(part, us, y, y2, M, N, splits, cu_count, stream);
 }
 
 // M > 128 where neither rule above applies: 192-row x 128-token tiles with
@@ -1206,6 +1220,31 @@ hipError_t launch_qgemm(int value_type, const uint8_t* w, uint32_t wbytes, void*
     case kQ6K: return launch_qgemm_m<kQ6K>(w, wbytes, workspace, workspace_bytes, y, M, N, K, cu_count, stream);
     default: return hipErrorInvalidValue;
     }
+}
+
+// Splits of the pair's one launch, or 0 where two launches serve it.
+static int pair_splits(int M, int N, int K, size_t workspace_bytes, int cu_count) {
+    const size_t part_off = align256((size_t)M * K * 2) + align256((size_t)M * 4);
+    if (M <= 128 || N % 256 != 0 || (uint64_t)(M + kTileTokMax) * (uint64_t)K * 2u >= (1ull << 32)) return 0;
+    if (M >= kTileWideM && use_tile(M, N, cu_count, 4, 9)) return 0;  // one matrix fills the CUs by itself
+    return wide256_splits(M, 2 * N, K, workspace_bytes > part_off ? workspace_bytes - part_off : 0, cu_count);
+}
+
+hipError_t launch_qgemm_pair(int value_type, const uint8_t* w0, const uint8_t* w1, uint32_t wbytes, void* workspace,
+                             size_t workspace_bytes, float* y0, float* y1, int M, int N, int K, int cu_count,
+                             hipStream_t stream) {
+    const int s = pair_splits(M, N, K, workspace_bytes, cu_count);
+    if (s > 0) {
+        switch (value_type) {
+        case kQ4K: return launch_tile_t<kQ4K, 4, 8>(workspace, w0, wbytes, y0, M, N, K, s, cu_count, stream, w1, y1);
+        case kQ5K: return launch_tile_t<kQ5K, 4, 8>(workspace, w0, wbytes, y0, M, N, K, s, cu_count, stream, w1, y1);
+        case kQ6K: return launch_tile_t<kQ6K, 4, 8>(workspace, w0, wbytes, y0, M, N, K, s, cu_count, stream, w1, y1);
+        default: return hipErrorInvalidValue;
+        }
+    }
+    hipError_t e = launch_qgemm(value_type, w0, wbytes, workspace, workspace_bytes, y0, M, N, K, cu_count, stream);
+    if (e != hipSuccess) return e;
+    return launch_qgemm(value_type, w1, wbytes, workspace, workspace_bytes, y1, M, N, K, cu_count, stream);
 }
 
 }  // namespace ribn_amd

@@ -582,8 +582,15 @@ hipError_t enqueue_prompt_chunk(ribn_amd_qwen3_decode* d, ribn_amd_kv_cache* cac
                    : ribn_amd::launch_act_f16_residual(d->p_hidden, d->p_y, L.attn_norm, c.epsilon, tokens,
                                                        (int)c.hidden, d->p_gemm, stream);
         if (e == hipSuccess && !last) e = prompt_gemm(d, L.attn_q, d->p_q, tokens, stream);
-        if (e == hipSuccess) e = prompt_gemm(d, L.attn_k, d->p_k, tokens, stream);
-        if (e == hipSuccess) e = prompt_gemm(d, L.attn_v, d->p_v, tokens, stream);
+        if (e == hipSuccess && L.attn_k->value_type == L.attn_v->value_type) {
+            e = ribn_amd::launch_qgemm_pair((int)L.attn_k->value_type, L.attn_k->data, L.attn_v->data,
+                                            (uint32_t)L.attn_k->encoded_bytes, d->p_gemm, d->p_gemm_bytes, d->p_k, d->p_v,
+                                            tokens, (int)L.attn_k->output_size, (int)L.attn_k->input_size,
+                                            d->ctx->cu_count, stream);
+        } else {
+            if (e == hipSuccess) e = prompt_gemm(d, L.attn_k, d->p_k, tokens, stream);
+            if (e == hipSuccess) e = prompt_gemm(d, L.attn_v, d->p_v, tokens, stream);
+        }
         if (e != hipSuccess) break;
         ribn_amd::PrefillAttnArgs a{};
         a.mem = descriptor(cache, nullptr);

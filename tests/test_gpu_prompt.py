@@ -368,3 +368,50 @@ def test_wide_chunk_attention(env, qh, kvh, p0, T):
         sc = (qd[:, h] @ kh.t().contiguous()) / 128 ** 0.5
         ref = (torch.softmax(sc.masked_fill(~seen, -np.inf), -1) @ vh).cpu().numpy()
         assert max_rel_err(got[:, h], ref) <= ATTN_TOL, h
+
+
+@pytest.mark.parametrize("t,kvh,T", [(12, 8, 300), (13, 8, 333), (14, 16, 257), (12, 8, 129)])
+def test_prompt_kv_pair(env, t, kvh, T):
+    """k and v of a prompt chunk in one paired matmul (and, at 129 tokens, the split it cannot fill):
+    the appended keys and values of a one-layer decoder against f64 products of the dequantised
+    weights, normwise within the f16 product's 1e-3 and the f16 cache's half unit, 2^-11."""
+    import torch
+    case(test="prompt_kv_pair", t=t, kvh=kvh, T=T)
+    E, ctx = env["E"], env["ctx"]
+    h, vocab, nkv = 2048, 320, kvh * 128
+    cfg = dict(layers=1, hidden=h, q_heads=16, kv_heads=kvh, head_dim=128, ffn=256, vocab=vocab, rope_base=1.0e6,
+               epsilon=1.0e-6)
+    store = E.AmdWeightStore(ctx)
+    enc, w = {}, {}
+    for i, (nm, ty, k, n) in enumerate((("token_embd", 12, h, vocab), ("output", 14, h, vocab), ("attn_q", 12, h, h),
+                                        ("attn_k", t, h, nkv), ("attn_v", t, h, nkv), ("attn_output", 12, h, h),
+                                        ("ffn_gate", 12, h, 256), ("ffn_up", 12, h, 256), ("ffn_down", 13, 256, h))):
+        enc[nm] = synth.kquant_numpy(ty, k, n, seed=900 + i + t, centered=True)
+        store.materialize_quantized(nm, [k, n], ty, enc[nm])
+        w[nm] = store.quantized_tensor(nm)
+    norms = {nm: synth.gamma_numpy(n, seed=950 + i) for i, (nm, n) in enumerate(
+        (("output_norm", h), ("attn_norm", h), ("ffn_norm", h), ("attn_q_norm", 128), ("attn_k_norm", 128)))}
+    dev = {nm: to_dev(v) for nm, v in norms.items()}
+    layer = {nm: w[nm] for nm in ("attn_q", "attn_k", "attn_v", "attn_output", "ffn_gate", "ffn_up", "ffn_down")}
+    layer.update({nm: dev[nm] for nm in ("attn_norm", "ffn_norm", "attn_q_norm", "attn_k_norm")})
+    conf = E.AmdQwen3Config(**cfg)
+    dec = E.AmdQwen3Decode(ctx, conf, w["token_embd"], w["output"], dev["output_norm"], [layer], 1)
+    cache = E.AmdKvCache(ctx, conf, T)
+    tokens = np.random.default_rng(T).integers(0, vocab, T)
+    dec.prefill_prompt(cache, tokens, 0)
+    ctx.synchronize()
+    got_k, got_v = (a.view(np.float16).astype(np.float64) for a in cache_arrays(env, cache, cfg)[0])
+
+    def rms(x, g):
+        return x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-6) * g.astype(np.float64)
+
+    x = O.dequantize_tensor(12, enc["token_embd"]).reshape(vocab, h)[tokens].astype(np.float64)
+    x = rms(x, norms["attn_norm"])
+    k, v = (x @ O.dequantize_tensor(t, enc[nm]).reshape(nkv, h).T.astype(np.float64) for nm in ("attn_k", "attn_v"))
+    k = rms(k.reshape(T, kvh, 128), norms["attn_k_norm"])
+    ang = np.arange(T)[:, None] * 1.0e6 ** (-np.arange(64) / 64.0)
+    c, s = np.cos(ang)[:, None], np.sin(ang)[:, None]
+    k = np.concatenate((k[..., :64] * c - k[..., 64:] * s, k[..., :64] * s + k[..., 64:] * c), -1)
+    for got, ref in ((got_k, k), (got_v, v.reshape(T, kvh, 128))):
+        assert max_rel_err(got.transpose(1, 0, 2), ref) <= 1e-3 + 2.0 ** -11
+    dec.close()

@@ -1471,9 +1471,9 @@ hipError_t launch_few(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
     }
 }
 
-// Three to eight members (one form for all: at three, 4-member groups still beat
-// the VALU rows, 6.6 against 7.5 us at 4096 rows): one workgroup per CU over the slice (or, SPLIT, over
-// the slices in proportion to their super-blocks).
+// Three to eight members (one form for all; four members of 4096 rows 7.5 us on
+// the VALU rows, 6.6 here; three use the four-member form): one workgroup per CU
+// over the slice (or, SPLIT, over the slices in proportion to their super-blocks).
 template <int T, int MG, int PRO, bool PAIR, bool SPLIT = false>
 hipError_t launch_many_instance(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
     constexpr int kRing = 2;

@@ -226,7 +226,7 @@ __device__ __forceinline__ uint4 funnel4(uint4 a, uint32_t t, uint32_t sh) {
 
 // Weights are dequantised in packed f16 (two per instruction, no conversion
 // instructions): a quant byte q becomes the f16 1024 + q (bits 0x6400 | q,
-// or 1024 + 16q for a high nibble left in place), and
+// or 1024 + 16q for a Q4_K high nibble left in place), and
 //   Q4_K/Q5_K: qs = fma(1024 + q, sc, -1024 sc) = q*sc exactly (every value
 //              involved is an f16 integer, q*sc <= 1953), then
 //              w = fma(qs, d, -f16(dmin*m)): one rounding of d*sc*q - dmin*m
@@ -255,23 +255,41 @@ __device__ __forceinline__ uint32_t f16_magic() {
     return k;
 }
 
-template <int T>
-__device__ __forceinline__ void tile_word(uint32_t x, uint32_t mask, uint32_t extra_a, uint32_t extra_b, half2_t s,
-                                          half2_t c, half2_t d, half2_t nb, uint32_t& oa, uint32_t& ob) {
+// Quant bytes (b0, b1, b2, b3) -> the f16 pairs 1024 + (b0, b1) and
+// 1024 + (b2, b3): one byte permute each, the 0x64 taken from a register.
+// (Masking each pair out of a permuted word and joining the 0x64 took five
+// instructions a word. Past the second, a VALU instruction beside an MFMA adds
+// its own four cycles, and the tile kernel has about four of them: now 3.3 for
+// Q5_K (4.3 before) and 3.9 for Q6_K (4.4). 2,047 tokens, activation stage
+// included: Q5_K 4096 -> 12288 296 -> 281 us, 12288 -> 4096 298 -> 286; Q6_K
+// 360 -> 333 and 340 -> 326; at 300 tokens 2 to 6%.)
+__device__ __forceinline__ void f16_pairs(uint32_t x, half2_t& a, half2_t& b) {
+    const uint32_t k = f16_magic();
+    a = as_h2(__builtin_amdgcn_perm(x, k, 0x01050104u));
+    b = as_h2(__builtin_amdgcn_perm(x, k, 0x01070106u));
+}
+
+// The same of a word of Q4_K nibbles in pair order, masked in place: the two
+// nibbles of a word share one permute, so this form is the shorter one there.
+__device__ __forceinline__ void nibble_pairs(uint32_t x, uint32_t mask, half2_t& a, half2_t& b) {
     const uint32_t xp = pair_order(x);
     const uint32_t k = f16_magic();
-    const half2_t pa = as_h2((xp & mask) | (extra_a | k));
-    const half2_t pb = as_h2(((xp >> 8) & mask) | (extra_b | k));
+    a = as_h2((xp & mask) | k);
+    b = as_h2(((xp >> 8) & mask) | k);
+}
+
+__device__ __forceinline__ void tile_word(half2_t pa, half2_t pb, half2_t s, half2_t c, half2_t d, half2_t nb,
+                                          uint32_t& oa, uint32_t& ob) {
     oa = as_u(__builtin_elementwise_fma(__builtin_elementwise_fma(pa, s, c), d, nb));
     ob = as_u(__builtin_elementwise_fma(__builtin_elementwise_fma(pb, s, c), d, nb));
 }
 
 __device__ __forceinline__ void tile_word6(uint32_t x, half2_t ahi, half2_t alo, uint32_t& oa, uint32_t& ob) {
-    const uint32_t xp = pair_order(x);
-    const uint32_t k = f16_magic();
+    half2_t pa, pb;
+    f16_pairs(x, pa, pb);
     const half2_t off = half2_t{(_Float16)-1056.0f, (_Float16)-1056.0f};
-    const half2_t qa = as_h2((xp & 0x003f003fu) | k) + off;
-    const half2_t qb = as_h2(((xp >> 8) & 0x003f003fu) | k) + off;
+    const half2_t qa = pa + off;
+    const half2_t qb = pb + off;
     oa = as_u(__builtin_elementwise_fma(qa, ahi, qa * alo));
     ob = as_u(__builtin_elementwise_fma(qb, ahi, qb * alo));
 }
@@ -281,8 +299,11 @@ __device__ __forceinline__ void tile_word6(uint32_t x, half2_t ahi, half2_t alo,
 __device__ __forceinline__ half8_t dequant8_qs(uint32_t lo, uint32_t hi, half2_t s, half2_t c, half2_t d,
                                                half2_t nb) {
     uint32_t o[4];
-    tile_word<kQ4K>(lo, 0x00ff00ffu, 0, 0, s, c, d, nb, o[0], o[1]);
-    tile_word<kQ4K>(hi, 0x00ff00ffu, 0, 0, s, c, d, nb, o[2], o[3]);
+    half2_t pa, pb;
+    f16_pairs(lo, pa, pb);
+    tile_word(pa, pb, s, c, d, nb, o[0], o[1]);
+    f16_pairs(hi, pa, pb);
+    tile_word(pa, pb, s, c, d, nb, o[2], o[3]);
     return __builtin_bit_cast(half8_t, uint4{o[0], o[1], o[2], o[3]});
 }
 
@@ -646,8 +667,9 @@ __device__ __forceinline__ void decode_sb(const SbW<T>& s, int q, SbDec<T>& o) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const float scf = (float)((sc[L] >> (8 * h)) & 0xffu);
-                o.s[L][h] = splat_h2(h ? scf * 0.0625f : scf);
-                o.c[L][h] = splat_h2(h ? -64.0f * scf : -1024.0f * scf);
+                const float up = T == kQ4K && h ? 0.0625f : 1.0f;  // a Q4_K high nibble stays 16x
+                o.s[L][h] = splat_h2(scf * up);
+                o.c[L][h] = splat_h2(-1024.0f * up * scf);
                 o.nb[L][h] = splat_h2(-(dmin * (float)((mn[L] >> (8 * h)) & 0xffu)));
             }
         }
@@ -671,9 +693,6 @@ __device__ __forceinline__ void decode_sb(const SbW<T>& s, int q, SbDec<T>& o) {
     }
 }
 
-// Four packed f16 weights from one word of quant bytes (elements j..j+3)
-// whose values, after `mask`, sit in the low bits of each byte (plus `extra`
-// bits already placed: the Q5_K high bit).
 // Chunk C's A fragment (8 f16 weights of the lane's row).
 template <int T, int C>
 __device__ __forceinline__ half8_t tile_chunk(const SbW<T>& s, const SbDec<T>& dec, int q) {
@@ -681,21 +700,20 @@ __device__ __forceinline__ half8_t tile_chunk(const SbW<T>& s, const SbDec<T>& d
     if constexpr (T == kQ4K || T == kQ5K) {
         constexpr int L = C >> 2, h = (C >> 1) & 1, p = C & 1;
         const uint4 P = L ? s.p1 : s.p0;
-        const uint32_t mask = h ? 0x00f000f0u : 0x000f000fu;
-        uint32_t ea0 = 0, eb0 = 0, ea1 = 0, eb1 = 0;
-        if constexpr (T == kQ5K) {
-            // bit g of each qh byte -> bit 4 (low nibble) or 8 (high nibble, 16x) of its f16 half
-            const int g = 4 * L + 2 * (q >> 1) + h;
-            const uint32_t hm = h ? 0x01000100u : 0x00100010u;
-            const int ra = (g + (h ? 24 : 28)) & 31, rb = (g + (h ? 0 : 4)) & 31;
-            const uint32_t q0 = pair_order(p ? s.qh.z : s.qh.x), q1 = pair_order(p ? s.qh.w : s.qh.y);
-            ea0 = __builtin_amdgcn_alignbit(q0, q0, ra) & hm;
-            eb0 = __builtin_amdgcn_alignbit(q0, q0, rb) & hm;
-            ea1 = __builtin_amdgcn_alignbit(q1, q1, ra) & hm;
-            eb1 = __builtin_amdgcn_alignbit(q1, q1, rb) & hm;
+        const uint32_t lo = p ? P.z : P.x, hi = p ? P.w : P.y;
+        half2_t pa, pb, pc, pd;
+        if constexpr (T == kQ4K) {
+            nibble_pairs(lo, h ? 0x00f000f0u : 0x000f000fu, pa, pb);
+            nibble_pairs(hi, h ? 0x00f000f0u : 0x000f000fu, pc, pd);
+        } else {
+            // bit g of each qh byte -> bit 4, in one rotate
+            const int ra = (4 * L + 2 * (q >> 1) + h + 28) & 31;
+            const uint32_t q0 = p ? s.qh.z : s.qh.x, q1 = p ? s.qh.w : s.qh.y;
+            f16_pairs(((lo >> (4 * h)) & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(q0, q0, ra) & 0x10101010u), pa, pb);
+            f16_pairs(((hi >> (4 * h)) & 0x0f0f0f0fu) | (__builtin_amdgcn_alignbit(q1, q1, ra) & 0x10101010u), pc, pd);
         }
-        tile_word<T>(p ? P.z : P.x, mask, ea0, eb0, dec.s[L][h], dec.c[L][h], dec.d, dec.nb[L][h], o[0], o[1]);
-        tile_word<T>(p ? P.w : P.y, mask, ea1, eb1, dec.s[L][h], dec.c[L][h], dec.d, dec.nb[L][h], o[2], o[3]);
+        tile_word(pa, pb, dec.s[L][h], dec.c[L][h], dec.d, dec.nb[L][h], o[0], o[1]);
+        tile_word(pc, pd, dec.s[L][h], dec.c[L][h], dec.d, dec.nb[L][h], o[2], o[3]);
     } else {
         constexpr int Q = C >> 1, p = C & 1;
         const uint4 W = (Q & 1) ? dec.lb : dec.la;

@@ -234,6 +234,161 @@ __device__ __forceinline__ void row_dot(const RowData<T>& d, int p, XF xf, SF sf
     }
 }
 
+// row_dot for gemv_f32_kernel's ring, the same operations in the same order. It
+// spells out what the helpers above compute, and Q6_K keeps two loops of one
+// trip, because the compiler's order of loads and conversions depends on both,
+// and the ring's rate on that order: through row_dot one member of Q6_K
+// 12288 -> 4096 took 11.8 us, without the two loops 11.3, as it stands 10.6; Q5_K
+// 12288 -> 4096 10.2 against 10.0. (Two members of Q6_K in one slice are faster
+// through row_dot, gate/up of 2048 -> 2 x 3072 8.7 against 9.1 us.)
+template <int T, int MT, class XF, class SF>
+__device__ __forceinline__ void ring_row_dot(const RowData<T>& row, int p, XF xf, SF sf, float (&part)[MT]) {
+    const RowData<T> d = row;
+    if constexpr (T == kQ4K || T == kQ5K) {
+        const uint4 h = d.h;
+        const float dd = half_bits_to_float(h.x & 0xffffu);
+        const float dmin = half_bits_to_float(h.x >> 16);
+        // six-bit scales / minima of all 8 groups, four per word (lib.rs:573-587)
+        const uint32_t lo_sc = h.y & 0x3f3f3f3fu;
+        const uint32_t lo_mn = h.z & 0x3f3f3f3fu;
+        const uint32_t hi_sc = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+        const uint32_t hi_mn = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
+        const uint32_t scw = (p < 2) ? lo_sc : hi_sc;
+        const uint32_t mnw = (p < 2) ? lo_mn : hi_mn;
+        const int sh = (p & 1) * 16;
+        // Q4_K quants enter as q * 2^-9 (see below): scales carry the 2^9, exactly
+        constexpr float kQScale = (T == kQ4K) ? 512.0f : 1.0f;
+        const float a0 = (dd * (float)((scw >> sh) & 0xffu)) * kQScale;
+        const float a1 = (dd * (float)((scw >> (sh + 8)) & 0xffu)) * kQScale;
+        const float b0 = dmin * (float)((mnw >> sh) & 0xffu);
+        const float b1 = dmin * (float)((mnw >> (sh + 8)) & 0xffu);
+        float sA[MT], sB[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) sA[m] = sB[m] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            // group A = 2p (low nibbles), group B = 2p+1 (high nibbles), 5th bit for Q5_K
+            float fa[4], fb[4];
+            const uint32_t qw[8] = {d.qa.x, d.qa.y, d.qa.z, d.qa.w, d.qb.x, d.qb.y, d.qb.z, d.qb.w};
+            uint32_t qa = qw[j] & 0x0f0f0f0fu;
+            uint32_t qb = (qw[j] >> 4) & 0x0f0f0f0fu;
+            if constexpr (T == kQ5K) {
+                const uint32_t hw[8] = {d.ha.x, d.ha.y, d.ha.z, d.ha.w, d.hb.x, d.hb.y, d.hb.z, d.hb.w};
+                qa |= ((hw[j] >> (2 * p)) & 0x01010101u) << 4;
+                qb |= ((hw[j] >> (2 * p + 1)) & 0x01010101u) << 4;
+            }
+            if constexpr (T == kQ4K) {
+                // Bytes 0..15 read as OCP E4M3 are exactly q * 2^-9: two
+                // quants per convert (the 2^9 is folded into the scales).
+                const auto a01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qa, false);
+                const auto a23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qa, true);
+                const auto b01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qb, false);
+                const auto b23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)qb, true);
+                fa[0] = a01[0];
+                fa[1] = a01[1];
+                fa[2] = a23[0];
+                fa[3] = a23[1];
+                fb[0] = b01[0];
+                fb[1] = b01[1];
+                fb[2] = b23[0];
+                fb[3] = b23[1];
+            } else {
+                qa = opaque(qa);
+                qb = opaque(qb);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    fa[t] = byte_f(qa, t);
+                    fb[t] = byte_f(qb, t);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const float4 xa = xf(m, j);
+                const float4 xb = xf(m, 8 + j);
+                sA[m] = __builtin_fmaf(fa[0], xa.x, sA[m]);
+                sA[m] = __builtin_fmaf(fa[1], xa.y, sA[m]);
+                sA[m] = __builtin_fmaf(fa[2], xa.z, sA[m]);
+                sA[m] = __builtin_fmaf(fa[3], xa.w, sA[m]);
+                sB[m] = __builtin_fmaf(fb[0], xb.x, sB[m]);
+                sB[m] = __builtin_fmaf(fb[1], xb.y, sB[m]);
+                sB[m] = __builtin_fmaf(fb[2], xb.z, sB[m]);
+                sB[m] = __builtin_fmaf(fb[3], xb.w, sB[m]);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const float xA = sf(m, 0), xB = sf(m, 1);
+            const float tA = __builtin_fmaf(a0, sA[m], -(b0 * xA));
+            const float tB = __builtin_fmaf(a1, sB[m], -(b1 * xB));
+            part[m] = tA + tB;
+        }
+    } else {
+        const int c = p >> 1, s = p & 1;
+        float a[4];
+        uint32_t law[4], lbw[4], qhw[4];
+#pragma unroll
+        for (int once = 0; once < 1; ++once) {
+            const uint32_t sh = d.shift;
+            const uint4 la = funnel(d.la, d.la_t, sh);
+            const uint4 lb = funnel(d.lb, d.lb_t, sh);
+            const uint4 qh = funnel(d.qh, d.qh_t, sh);
+            const uint4 sc = funnel(d.sc, d.sc_t, sh);  // int8 scales
+            const float dd = half_bits_to_float(d.d16);
+            const uint32_t w0 = c ? sc.z : sc.x;  // scales 8c+0..8c+3
+            const uint32_t w1 = c ? sc.w : sc.y;  // scales 8c+4..8c+7
+            a[0] = dd * (float)(int8_t)((w0 >> (8 * s)) & 0xffu);
+            a[1] = dd * (float)(int8_t)((w0 >> (8 * (2 + s))) & 0xffu);
+            a[2] = dd * (float)(int8_t)((w1 >> (8 * s)) & 0xffu);
+            a[3] = dd * (float)(int8_t)((w1 >> (8 * (2 + s))) & 0xffu);
+            law[0] = la.x; law[1] = la.y; law[2] = la.z; law[3] = la.w;
+            lbw[0] = lb.x; lbw[1] = lb.y; lbw[2] = lb.z; lbw[3] = lb.w;
+            qhw[0] = qh.x; qhw[1] = qh.y; qhw[2] = qh.z; qhw[3] = qh.w;
+        }
+        // One 16-element group v at a time: quants 0..63 of group v are
+        // element 16v + 4j + t of the lane's record (the -32 offset enters
+        // through X_v).
+        float acc[MT];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            float sv[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) sv[m] = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float f[4];
+                uint32_t q;
+                const uint32_t lw = (v & 1) ? lbw[j] : law[j];
+                if (v == 0) q = (lw & 0x0f0f0f0fu) | ((qhw[j] << 4) & 0x30303030u);
+                else if (v == 1) q = (lw & 0x0f0f0f0fu) | ((qhw[j] << 2) & 0x30303030u);
+                else if (v == 2) q = ((lw >> 4) & 0x0f0f0f0fu) | (qhw[j] & 0x30303030u);
+                else q = ((lw >> 4) & 0x0f0f0f0fu) | ((qhw[j] >> 2) & 0x30303030u);
+                q = opaque(q);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) f[t] = byte_f(q, t);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const float4 xv = xf(m, 4 * v + j);
+                    sv[m] = __builtin_fmaf(f[0], xv.x, sv[m]);
+                    sv[m] = __builtin_fmaf(f[1], xv.y, sv[m]);
+                    sv[m] = __builtin_fmaf(f[2], xv.z, sv[m]);
+                    sv[m] = __builtin_fmaf(f[3], xv.w, sv[m]);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const float x32 = 32.0f * sf(m, v);  // exact
+#pragma unroll
+                for (int once = 0; once < 1; ++once) {
+                    const float t = a[v] * (sv[m] - x32);
+                    acc[m] = (v == 0) ? t : acc[m] + t;
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) part[m] = acc[m];
+    }
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------ kernel
@@ -504,7 +659,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
             if (r % GROUP == 0) read_rec(cslice);
         }
         float part[MT];
-        row_dot<T, MT>(d, p, xf, sf, part);
+        if constexpr (T == kQ6K && MT == 2 && ONE_SLICE) {
+            row_dot<T, MT>(d, p, xf, sf, part);
+        } else {
+            ring_row_dot<T, MT>(d, p, xf, sf, part);
+        }
         const int ai = ONE_SLICE ? 0 : r % GROUP;
         const int row = ONE_SLICE ? crow : crow + r % GROUP;
         const bool last = ONE_SLICE || cslice == slices - 1;

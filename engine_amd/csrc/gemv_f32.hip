@@ -1591,26 +1591,54 @@ hipError_t launch_slices(const WaveGemvArgs& a, int cu_count, hipStream_t stream
     return hipGetLastError();
 }
 
+// K above 4096, one or two members: whether pairs of rows over all slices (a wave
+// rereads the slices' records for every pair) beat the units of
+// gemv_f32_slices_kernel. A wave takes ceil(rows / 16 per CU) pairs, `pair_units`
+// units. Plain products: the slices form costs about as much more a launch as two
+// units take, so it has to save two, or one where two members make the rereads
+// dearer (Q4_K, and a short last slice after one whole slice); longer launches
+// hide it. With a SwiGLU pairs are faster only where nothing is saved over four
+// slices (three for one member of Q5_K and Q6_K), with an RMSNorm nowhere. Pairs time / slices time over K 4608 .. 16384 and 2 .. 68 rows a CU,
+// Q4_K / Q5_K / Q6_K:
+//   plain, one member, two or more units saved 1.04-1.7 / 1.02-1.8 / 1.03-1.7, one
+//   saved 0.86-0.99 / 0.94-1.03 / 0.88-1.04, none 0.84-1.13 (0.91-0.99 up to 32 rows
+//   a CU; two whole slices 0.95-0.99 at 48); e.g. us, Q4_K: 5120 at 3072 and 4096 rows
+//   6.9 / 6.1 and 7.0 / 7.6; 8192 at 2560 rows 6.3 / 7.0; 12288 at 2048, 2560 and 5120
+//   rows 8.1 / 7.4, 8.2 / 9.0 and 13.8 / 11.3
+//   SwiGLU, K up to 9728 1.03-1.7, 12288 0.96-1.5, 16384 at 13 to 16 rows a CU 0.92-0.97
+//   RMSNorm 0.98-1.7
+template <int T, int MT, int PRO>
+bool pairs_form(const WaveGemvArgs& a, int cu_count) {
+    const long long per_cu = ((long long)a.total_rows + cu_count - 1) / cu_count;
+    const int nb = a.K >> 8, slices = (nb + 15) >> 4;
+    const long long quad_units = 4 * (slices - 1) + 4 / unit_rows(nb - 16 * (slices - 1));
+    const long long slice_units = ((per_cu + 3) / 4 * quad_units + kSliceWaves - 1) / kSliceWaves;
+    const long long pair_units = 2 * slices * ((per_cu + 15) / 16);
+    if (PRO == kProSwiglu) {
+        return per_cu <= 16 && pair_units <= slice_units && (slices > 3 || (slices == 3 && MT == 1 && T != kQ4K));
+    }
+    if (per_cu > (slices == 2 ? 48 : 32)) return false;
+    const int save = MT == 2 && (T == kQ4K || (slices == 2 && unit_rows(nb - 16) > 1)) ? 1 : 2;
+    return pair_units - slice_units < save;
+}
+
 // One or two members.
 template <int T, int MT, int PRO, bool ONE_SLICE, bool PAIR = false>
 hipError_t launch_few(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
     if constexpr (!ONE_SLICE) {
-        // One pair of rows per wave over (nearly) every wave is where reading
-        // the records once a pair costs least: up to 16 rows per CU that form
-        // stays (Q4_K, one member, us, pairs / slices: K 5120 at 3072, 4096,
-        // 5120 rows 6.9 / 6.3, 7.1 / 7.7, 10.7 / 8.4; K 12288 at 2048, 3072, 4096,
-        // 5120 rows 8.9 / 8.2, 9.6 / 10.2, 10.2 / 11.2, 15.7 / 13.1).
-        const long long from = (a.K <= 2 * kSliceElems ? 15LL : 11LL) * cu_count;
-        if (a.total_rows > from && a.total_rows <= 16LL * cu_count) {
-            return F32Instance<T, MT, PRO, false, 2, 8, 2>::launch(a, cu_count, 1, stream);
+        if constexpr (PRO != kProNorm) {
+            if (pairs_form<T, MT, PRO>(a, cu_count)) return F32Instance<T, MT, PRO, false, 2, 8, 2>::launch(a, cu_count, 1, stream);
         }
         return launch_slices<T, MT, PRO, true>(a, cu_count, stream);
     } else {
         // Short rows: several to a unit, where the launch is long enough for it
-        // (Q4_K, one member, us, one row / several: K 1024 at 4096, 5120, 12288
-        // rows 4.2 / 4.6, 5.0 / 4.7, 7.0 / 5.7; K 2048 at 8192, 12288, 17408 rows
-        // 5.6 / 5.9, 7.8 / 7.5, 9.8 / 8.7).
-        if (a.total_rows > (a.K <= 1024 ? 16LL : 40LL) * cu_count && a.K <= 2048) {
+        // (us, one member, one row / several: Q4_K 1024 at 4096, 5120, 12288
+        // rows 4.2 / 4.6, 5.0 / 4.7, 7.0 / 5.7; 1536 at 10240, 10496, 16384 rows
+        // 6.2 / 6.2, 6.4 / 6.3, 8.1 / 7.2; 2048 at 10496, 12288, 14336 rows 6.4 / 6.8,
+        // 6.7 / 6.9, 7.7 / 7.5, with an RMSNorm 7.0 / 7.0, 7.2 / 7.1, 8.0 / 7.7; two
+        // members of K 1536 and 2048 at 10496 rows 1.10-1.15 times as fast).
+        const bool late = T == kQ4K && MT == 1 && PRO != kProNorm && a.K > 1536;
+        if (a.total_rows > (a.K <= 1024 ? 16LL : late ? 48LL : 40LL) * cu_count && a.K <= 2048) {
             return launch_slices<T, MT, PRO, false, PAIR>(a, cu_count, stream);
         }
         const long long per_cu = ((long long)a.total_rows + cu_count - 1) / cu_count;

@@ -785,3 +785,40 @@ def test_slices_form_gate_up_pairs(env, t, blocks, n):
         kern.execute_rms_norm(w, to_dev(x[0]), gamma, 1e-6, y, 1)
         parts.append(to_host(y, env["ctx"]))
     assert max_rel_err(outs[0][0], O.swiglu(parts[0], parts[1])) <= 1e-6  # expf's last bits
+
+
+@pytest.mark.parametrize("t,blocks,at,members,pro", [
+    (12, 20, 3072, 1, ""), (14, 32, 2048, 1, ""), (12, 32, 2048, 2, ""), (13, 38, 3072, 1, ""), (14, 48, 4096, 2, ""),
+    (12, 32, 12288, 1, ""), (14, 48, 3072, 1, "swiglu"), (13, 64, 4096, 2, "swiglu"), (12, 64, 3072, 2, "norm"),
+    (12, 8, 12288, 1, ""), (13, 8, 10240, 2, ""), (14, 3, 4096, 1, "norm")])
+def test_few_member_dispatch_lines(env, t, blocks, at, members, pro):
+    """One and two members on both sides of the lines between the row-pair, slices and short-row forms
+    (on 256 CUs): `at` rows and five more of the same weight give the same bits in the common rows,
+    and the first row is within the f32 bar of the oracle."""
+    check_dispatch_line(env, t, blocks, at, members, pro)
+
+
+def check_dispatch_line(env, t, blocks, at, members, pro):
+    k, n = 256 * blocks, at + 5
+    print_case(test="dispatch_line", t=t, k=k, at=at, members=members, pro=pro)
+    enc = synth.kquant_numpy(t, k, n, seed=k + at)
+    x = synth.activations_numpy(k, members, seed=blocks)
+    up = synth.activations_numpy(k, members, seed=blocks + 1)
+    gamma = synth.gamma_numpy(k, seed=blocks)
+    kern = env["k"][t]
+    got = []
+    for rows in (at, n):
+        w = upload(env, t, k, rows, enc[:len(enc) // n * rows])
+        y = empty_dev(members * rows)
+        if pro == "swiglu":
+            kern.execute_fused(w, to_dev(x.reshape(-1)), y, members, up=to_dev(up.reshape(-1)))
+        else:
+            kern.execute_group([w], to_dev(x.reshape(-1)), [y], members, gamma=to_dev(gamma) if pro == "norm" else None, epsilon=1e-6)
+        got.append(to_host(y, env["ctx"]).reshape(members, rows))
+    assert np.array_equal(got[0].view(np.uint32), got[1][:, :at].view(np.uint32))
+    for m in range(members):
+        xin = {"norm": lambda: O.rms_norm_raw(x[m], gamma, 1e-6), "swiglu": lambda: O.swiglu(x[m], up[m]), "": lambda: x[m]}[pro]()
+        # the bar is relative to the largest output: take 64 rows from both ends
+        for rows in (slice(0, 64), slice(n - 64, n)):
+            want = O.quant_gemv(t, enc[len(enc) // n * rows.start:len(enc) // n * rows.stop], k, 64, xin, threads=8)
+            assert max_rel_err(got[1][m, rows], want) <= F32_RTOL

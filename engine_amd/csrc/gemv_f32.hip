@@ -1735,12 +1735,31 @@ hipError_t launch_type(const WaveGemvArgs& a, int cu_count, hipStream_t stream) 
     return launch_plain<T, kProPlain>(a, cu_count, stream);
 }
 
+// One member, K above kWaveMaxK: whether one launch of the slices form, whose
+// workgroups stage all of K, beats a workgroup per slice and the reduction. Past
+// five slices staging costs more than the second launch where a workgroup has
+// one short run of units, or (Q4_K, and Q5_K of seven slices on) more than a few.
+// Split time / one launch, Q4_K / Q5_K / Q6_K: K 16640 .. 17408 at 1 and 2 rows a CU
+// 1.06-1.11 / 0.95-1.02 / 0.97-1.01, more 1.00-1.09 / 1.01-1.07 / 1.00-1.10 (Q6_K at 14
+// and 16 rows a CU 0.90-1.02; at K 17408 itself also 0.90 at 32 and 0.96 at 40); K 18432
+// .. 24576 at 1 and 2 rows a CU 1.01-1.09 / 0.94-0.98 / 0.94-0.97, 4 to 16 rows
+// 0.99-1.13, more 0.94-1.03 / 0.96-1.10 / 1.00-1.07; K 28672 and 32768 at 1 and 2 rows
+// 0.85-0.92, 4 and 8 rows 0.98-1.07, 12 and more 0.92-0.98 / 0.94-1.05 / 0.99-1.05.
+template <int T>
+bool one_launch_long_k(const WaveGemvArgs& a, int cu_count) {
+    if (a.K > 2 * kWaveMaxK) return false;
+    const long long per_cu = ((long long)a.total_rows + cu_count - 1) / cu_count;
+    if (a.K <= 17408) return T == kQ4K || (per_cu > 2 && (T == kQ5K || per_cu <= 12 || per_cu > 16));
+    const bool any_longer = T == kQ6K || (T == kQ5K && a.K <= 24576);
+    return per_cu > 2 && (any_longer || per_cu <= (a.K <= 24576 ? 16 : 8));
+}
+
 // Members over a K of several slices: one workgroup per (row range, slice),
 // then the ordered slice reduction. One member (a K beyond kWaveMaxK) keeps
 // its records in VGPRs, as the one-launch form does.
 template <int T>
 hipError_t launch_split(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
-    if (a.members == 1 && a.K <= 2 * kWaveMaxK) return launch_slices<T, 1, kProPlain, true>(a, cu_count, stream);
+    if (a.members == 1 && one_launch_long_k<T>(a, cu_count)) return launch_slices<T, 1, kProPlain, true>(a, cu_count, stream);
     hipError_t e = (a.members == 1)
                        ? F32Instance<T, 1, kProPlain, true, 3, 8, 1, false, true>::launch(a, cu_count, 1, stream)
                    : a.gamma != nullptr ? launch_many<T, kProNorm, false, true>(a, cu_count, stream)

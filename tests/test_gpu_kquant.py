@@ -822,3 +822,10 @@ def check_dispatch_line(env, t, blocks, at, members, pro):
         for rows in (slice(0, 64), slice(n - 64, n)):
             want = O.quant_gemv(t, enc[len(enc) // n * rows.start:len(enc) // n * rows.stop], k, 64, xin, threads=8)
             assert max_rel_err(got[1][m, rows], want) <= F32_RTOL
+
+
+@pytest.mark.parametrize("t,blocks,at", [(12, 112, 512), (13, 68, 512), (14, 68, 3072), (14, 66, 4096), (12, 80, 4096),
+                                         (13, 100, 2048)])
+def test_long_k_dispatch_lines(env, t, blocks, at):
+    """As above for one member of K beyond 16384, between one launch and the slice split."""
+    check_dispatch_line(env, t, blocks, at, 1, "")

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_f32_kernel(WaveGemvArgs args)
     constexpr int BB = BlockTraits<T>::bytes;
     constexpr int NBMAX = ONE_SLICE ? 16 : kF32Blocks;
     constexpr int NBW = (NBMAX + WAVES - 1) / WAVES;  // staging blocks per wave
-    extern __shared__ __attribute__((aligned(16))) float xs[];                     // [MT][slices][64 records][STRIDE]
+    extern __shared__ __attribute__((aligned(16))) float xs[];  // [MT][slices][64 records][STRIDE]
     __shared__ float ssq_s[NORM ? MT : 1][NORM ? NBMAX : 1];
 
     const int lane = threadIdx.x & 63;
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(kSliceWaves * 64) void gemv_f32_slices_kernel(WaveG
     constexpr int WAVES = kSliceWaves;
     constexpr int NBMAX = MULTI ? (MT == 1 ? 2 : 1) * kF32Blocks : 8;
     constexpr int NBW = MULTI ? 6 : 1;                // blocks a wave stages at a time
-    extern __shared__ __attribute__((aligned(16))) float xs[];                     // [MT][slices][64 records][STRIDE], then the slice totals
+    extern __shared__ __attribute__((aligned(16))) float xs[];  // [MT][slices][64 records][STRIDE], then the slice totals
     __shared__ float ssq_s[NORM ? MT : 1][NORM ? NBMAX : 1];
     __shared__ float inv_s[MT];
 
@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(kManyWaves * 64) void gemv_f32_many_kernel(WaveGemv
     constexpr int MT = 4 * MG;
     constexpr int BB = BlockTraits<T>::bytes;
     constexpr int NBW = 16 / kManyWaves;  // staging blocks per wave
-    extern __shared__ __attribute__((aligned(16))) float xs[];         // [MT][64 records][68] (member stride kManyStride), then the units' block sums
+    extern __shared__ __attribute__((aligned(16))) float xs[];  // [MT][64 records][68] (member stride kManyStride), then the units' block sums
     __shared__ float ssq_s[NORM && !SPLIT ? MT : 1][NORM && !SPLIT ? 16 : 1];
     __shared__ float inv_s[MT];
 
@@ -1524,10 +1524,13 @@ std::atomic<int> F32Instance<T, MT, PRO, ONE_SLICE, NBUF, WAVES, GROUP, PAIR, SP
 // y[m][row] (+)= ((P_0 + P_1) + P_2) ... over the slices of a SPLIT launch,
 // in slice order, times the RMSNorm factor: the slice totals of the one-launch
 // form, added the same way.
+// (NORM is a template argument: with a branch on args.gamma the plain reduction
+// was longer, one member of Q6_K 24576 -> 256 8.8 instead of 8.1 us.)
+template <bool NORM>
 __global__ __launch_bounds__(256) void f32_split_reduce_kernel(WaveGemvArgs a, int slices) {
     const int total = a.members * a.total_rows;
-    __shared__ float inv_s[kWaveMaxMembers];
-    if (a.gamma != nullptr) {
+    __shared__ float inv_s[NORM ? kWaveMaxMembers : 1];
+    if constexpr (NORM) {
         const int nb = a.K >> 8;
         if ((int)threadIdx.x < a.members) {
             const float* ssq = a.partial + (size_t)slices * total + (size_t)threadIdx.x * nb;
@@ -1542,7 +1545,7 @@ __global__ __launch_bounds__(256) void f32_split_reduce_kernel(WaveGemvArgs a, i
         const int row = i - m * a.total_rows;
         float t = a.partial[(size_t)m * a.total_rows + row];
         for (int s = 1; s < slices; ++s) t = t + a.partial[((size_t)s * a.members + m) * a.total_rows + row];
-        if (a.gamma != nullptr) t = t * inv_s[m];
+        if constexpr (NORM) t = t * inv_s[m];
         int mat = 0, start = 0;
         for (int g = 0; g + 1 < a.count; ++g) {
             if (row >= a.rows_end[g]) {
@@ -1768,7 +1771,11 @@ hipError_t launch_split(const WaveGemvArgs& a, int cu_count, hipStream_t stream)
     const int slices = ((a.K >> 8) + 15) >> 4;
     const long long total = (long long)a.members * a.total_rows;
     const unsigned grid = (unsigned)std::min<long long>((total + 255) / 256, (long long)cu_count * 4);
-    hipLaunchKernelGGL(f32_split_reduce_kernel, dim3(grid), dim3(256), 0, stream, a, slices);
+    if (a.gamma != nullptr) {
+        hipLaunchKernelGGL(f32_split_reduce_kernel<true>, dim3(grid), dim3(256), 0, stream, a, slices);
+    } else {
+        hipLaunchKernelGGL(f32_split_reduce_kernel<false>, dim3(grid), dim3(256), 0, stream, a, slices);
+    }
     return hipGetLastError();
 }
 

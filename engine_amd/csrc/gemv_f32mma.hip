@@ -991,6 +991,27 @@ F32MmaShape f32mma_shape_r(const F32MmaShape& one, int tiles, int R, int cu_coun
     return {w, one.splits, one.split_blocks, (units + w - 1) / w};
 }
 
+// The one-wave kernels, instantiated here so that they lie together in the code
+// object, before the two-wave ones that launch_shape would put between them. A
+// layer's kernels (56 KB of code at 16 members) about fill the instruction cache
+// that two CUs share, and their places decide what stays in it between launches:
+// six FFN layers at 16 members 291.6 us with the two-wave kernels between, 288.2
+// without (288.2 before there were any), the instructions of each unchanged.
+#define RIBN_ONE_WAVE_KERNELS(T, MT)                                                                                     \
+    template __global__ void f32mma_gemv_kernel<T, 2, MT, true, lds_slots<T, MT>(), ring_depth<T, 2, MT>(), 1>(F32MmaArgs); \
+    template __global__ void f32mma_gemv_kernel<T, 1, MT, false, lds_slots<T, MT>(), ring_depth<T, 1, MT>(), 1>(F32MmaArgs);
+RIBN_ONE_WAVE_KERNELS(kQ4K, 1)
+RIBN_ONE_WAVE_KERNELS(kQ4K, 2)
+RIBN_ONE_WAVE_KERNELS(kQ4K, 3)
+RIBN_ONE_WAVE_KERNELS(kQ4K, 4)
+RIBN_ONE_WAVE_KERNELS(kQ5K, 1)
+RIBN_ONE_WAVE_KERNELS(kQ5K, 2)
+RIBN_ONE_WAVE_KERNELS(kQ5K, 3)
+RIBN_ONE_WAVE_KERNELS(kQ5K, 4)
+RIBN_ONE_WAVE_KERNELS(kQ6K, 1)
+RIBN_ONE_WAVE_KERNELS(kQ6K, 2)
+#undef RIBN_ONE_WAVE_KERNELS
+
 template <int T, int R, int MT, bool PAIR>
 hipError_t launch_shape(F32MmaArgs a, const F32MmaShape& sh, hipStream_t stream) {
     a.splits = sh.splits;

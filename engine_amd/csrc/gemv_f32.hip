@@ -1097,13 +1097,16 @@ __global__ __launch_bounds__(kSliceWaves * 64) void gemv_f32_slices_kernel(WaveG
 // (r0 + r1) + (r2 + r3) through LDS, where the records were; one barrier per
 // kManyItems units.
 //
-// Measured (us, against rows through VALU FMAs with the records in LDS): 8
-// members, K 4096: Q4_K 4096 / 24576 / 98304 rows 10.9 / 38.3 / 134.6 -> 9.6 /
-// 30.7 / 105.4; Q5_K 24576 rows 42.7 -> 33.6; Q6_K 50.2 -> 38.7; 4 members, Q4_K
-// 24576 rows 26.1 -> 21.4. What bounds it: with the weights in cache 26.9 us, so
-// the f32 multiply-adds and the conversions; an MFMA takes 4.5 ns of a SIMD. A
-// ring of four units, two workgroups per CU (4 members), and weights loaded as
-// whole rows through an LDS slab were level or slower.
+// Measured (us a call over distinct weights, against rows through VALU FMAs with
+// the records in LDS), 8 members, K 4096 at 256 / 4096 / 12288 rows: Q4_K 9.5 / 9.9 /
+// 20.4 -> 7.2 / 9.4 / 16.1; Q5_K 10.0 / 10.7 / 21.3 -> 7.6 / 10.4 / 17.9; Q6_K 12.5 /
+// 13.2 / 26.0 -> 8.3 / 11.5 / 19.9; 4 members, Q4_K 6.3 / 6.6 / 13.5 -> 5.1 / 6.5 / 10.7.
+// (Slower in one place: Q5_K, 3 or 4 members, two units a wave, 4096 rows 7.1 -> 7.6:
+// the second unit runs the loop's code cold.) What bounds it: with the weights in
+// cache 26.9 us of Q4_K 4096 -> 24576's 30.7, so the f32 multiply-adds and the
+// conversions; an MFMA takes 4.5 ns of a SIMD. A ring of four units, two
+// workgroups per CU (4 members), and weights loaded as whole rows through an LDS
+// slab were level or slower.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kManyWaves = 8;
@@ -1116,17 +1119,18 @@ __device__ __forceinline__ float dpp_shift_add(float v) {
     return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// part[m] = this lane's share of its row . x_m (m = 0 .. 4 MG - 1): rows_dot's
+// part[m] = this lane's share of its row . x_m (m = 0 .. 4 MG - 1): row_dot's
 // operation sequence per (row, member), the FMAs on the matrix cores.
 template <int T, int MG>
 __device__ __forceinline__ void unit_dot(const RowData<T>& d, int p, const float4 (&x)[MG][16], const float (&xg)[MG][4],
                                          float (&part)[4 * MG]) {
-    constexpr int CH = 8;  // dwords of quants per run
+    constexpr int CH = T == kQ5K && MG == 2 ? 4 : 8;  // dwords of quants per run (of two groups)
     auto mac = [](float xv, float q, f32x4 s) { return __builtin_amdgcn_mfma_f32_4x4x1f32(xv, q, s, 0, 0, 0); };
-    // Quants are converted in runs, then multiplied in runs: a VALU instruction
-    // between two MFMAs costs about 1 ns more than one after another VALU
-    // instruction (8 members, Q4_K 4096 -> 98304: 122 us alternating, 106 in
-    // runs of 32 quants). The minimum terms m * X run as one more MFMA each.
+    // Quants are converted in runs, then multiplied in runs: 64 (CH dwords of two
+    // groups) for Q4_K and Q5_K, 32 for Q5_K at 5 to 8 members and Q6_K at 3 and 4, 16
+    // for Q6_K at 5 to 8. Q5_K, 8 members, 4096 -> 12288, 64 / 32: 18.5 / 17.6 us, 12288
+    // -> 4096 24.3 / 22.3; Q4_K level, runs of 8 too. The minimum terms m * X run
+    // as one more MFMA each.
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     if constexpr (T == kQ4K || T == kQ5K) {
         float a0, a1, b0, b1;
@@ -1230,7 +1234,7 @@ __device__ __forceinline__ void unit_dot(const RowData<T>& d, int p, const float
 template <int T, int MG, int PRO, int NBUF, bool PAIR, bool SPLIT>
 __global__ __launch_bounds__(kManyWaves * 64) void gemv_f32_many_kernel(WaveGemvArgs args, int wgs) {
     static_assert(kManyItems % NBUF == 0, "whole ring passes between barriers");
-    static_assert(!PAIR || NBUF % 2 == 0, "pairs are whole ring slots");
+    static_assert(!PAIR || NBUF == 2, "pairs are whole rings");
     static_assert(!SPLIT || !PAIR, "slice splits store slice totals");
     constexpr bool NORM = PRO == kProNorm;
     constexpr int MT = 4 * MG;
@@ -1445,25 +1449,36 @@ __global__ __launch_bounds__(kManyWaves * 64) void gemv_f32_many_kernel(WaveGemv
         }
     };
 
+    // Item c0 + k from its ring slot, which then takes the item NBUF ahead (a
+    // wave's last item takes none: a load there would make every ring pass wait
+    // for both slots).
+    auto reduce_item = [&](RowData<T>& d, int c0, int k, auto refill) {
+        float part[MT];
+        unit_dot<T, MG>(d, p, x, xg, part);
+        if constexpr (decltype(refill)::value) load_item(d, c0 + k + NBUF);
+        // a block's four records: ((0 + 1) + (2 + 3)), in the block's first quad
+#pragma unroll
+        for (int m = 0; m < MT; ++m) part[m] = dpp_shift_add<0x108>(dpp_shift_add<0x104>(part[m]));  // row_shl 4, 8
+        if ((lane & 12) == 0 && set < sets) {
+            float* dst = xs + k * kItemSums + wave * kWaveSums + (4 * (lane >> 4) + (lane & 3)) * MT;
+#pragma unroll
+            for (int g = 0; g < MG; ++g)
+                *reinterpret_cast<float4*>(dst + 4 * g) =
+                    float4{part[4 * g], part[4 * g + 1], part[4 * g + 2], part[4 * g + 3]};
+        }
+    };
     for (int c0 = 0; c0 < items; c0 += kManyItems) {
         const int count = min(kManyItems, items - c0);
-        for (int k0 = 0; k0 < count; k0 += NBUF) {
+        int k0 = 0;
+        for (; k0 + NBUF <= count; k0 += NBUF) {
 #pragma unroll
-            for (int r = 0; r < NBUF; ++r) {
-                float part[MT];
-                unit_dot<T, MG>(ring[r], p, x, xg, part);
-                load_item(ring[r], c0 + k0 + r + NBUF);
-                // a block's four records: ((0 + 1) + (2 + 3)), in the block's first quad
+            for (int r = 0; r < NBUF; ++r) reduce_item(ring[r], c0, k0 + r, std::true_type{});
+        }
+        // a wave's last items, where they are no whole ring (pairs are)
+        if constexpr (!PAIR) {
 #pragma unroll
-                for (int m = 0; m < MT; ++m) part[m] = dpp_shift_add<0x108>(dpp_shift_add<0x104>(part[m]));  // row_shl 4, 8
-                if ((lane & 12) == 0 && set < sets) {
-                    float* dst = xs + (k0 + r) * kItemSums + wave * kWaveSums + (4 * (lane >> 4) + (lane & 3)) * MT;
-#pragma unroll
-                    for (int g = 0; g < MG; ++g)
-                        *reinterpret_cast<float4*>(dst + 4 * g) =
-                            float4{part[4 * g], part[4 * g + 1], part[4 * g + 2], part[4 * g + 3]};
-                }
-            }
+            for (int r = 0; r + 1 < NBUF; ++r)
+                if (k0 + r < count) reduce_item(ring[r], c0, k0 + r, std::false_type{});
         }
         __syncthreads();
         finish(c0, count);

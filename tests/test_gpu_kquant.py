@@ -829,3 +829,12 @@ def check_dispatch_line(env, t, blocks, at, members, pro):
 def test_long_k_dispatch_lines(env, t, blocks, at):
     """As above for one member of K beyond 16384, between one launch and the slice split."""
     check_dispatch_line(env, t, blocks, at, 1, "")
+
+
+@pytest.mark.parametrize("t,blocks,ns,members,norm", [
+    (12, 16, (6150,), 8, False), (13, 16, (6141,), 4, True), (14, 16, (2050, 4100), 5, False), (13, 20, (3100,), 8, False),
+    (14, 4, (8200,), 3, True)])
+def test_many_members_odd_items(env, t, blocks, ns, members, norm):
+    """3..8 members where a wave's units are no whole ring (three of them, or one and more by
+    workgroup), with the checks of the edges test."""
+    test_many_members_edges_bit_identical(env, t, blocks, ns, members, norm)

@@ -646,6 +646,33 @@ constexpr int kPfKeys = 64;              // keys per block
 constexpr int kPfVRow = kPfKeys + 4;     // LDS V^T row (halfs): 136 B
 constexpr float kPfLazy = 15.0f;         // log2 headroom of the lazy softmax rescale
 
+// Values that are infinite or NaN. A key past a token's position has probability
+// 0, but 0 * inf is NaN, so in blocks with such keys (those from a workgroup's
+// first position on) non-finite values are staged as zeros and added to the
+// tokens that attend them after the key loop. (Finding them costs 50 instructions a
+// thread in those blocks.)
+// One bit (15 and 31) per half of w that is not finite.
+__device__ __forceinline__ uint32_t nonfinite_halfs(uint32_t w) { return ((w & 0x7fff7fffu) + 0x04000400u) & 0x80008000u; }
+
+// A V unit's 16 words with their non-finite halfs zero; whether there were any.
+__device__ __forceinline__ bool drop_nonfinite(uint4 (&vp)[4]) {
+    uint32_t bad = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bad |= nonfinite_halfs(vp[r].x) | nonfinite_halfs(vp[r].y) | nonfinite_halfs(vp[r].z) | nonfinite_halfs(vp[r].w);
+    if (bad == 0) return false;
+    auto finite = [](uint32_t w) { return w & ~((nonfinite_halfs(w) >> 15) * 0xffffu); };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) vp[r] = make_uint4(finite(vp[r].x), finite(vp[r].y), finite(vp[r].z), finite(vp[r].w));
+    return true;
+}
+
+// The non-finite ones of four values (two words of halfs), zeros elsewhere.
+__device__ __forceinline__ float4 nonfinite_values(uint2 w) {
+    const uint32_t bx = nonfinite_halfs(w.x), by = nonfinite_halfs(w.y);
+    return make_float4(bx & 0x8000u ? half_bits_to_float(w.x & 0xffffu) : 0.f, bx >> 31 ? half_bits_to_float(w.x >> 16) : 0.f,
+                       by & 0x8000u ? half_bits_to_float(w.y & 0xffffu) : 0.f, by >> 31 ? half_bits_to_float(w.y >> 16) : 0.f);
+}
+
 template <int QPK>
 __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(PrefillAttnArgs a) {
     constexpr int W = QPK < 4 ? 4 : QPK;  // waves
@@ -655,6 +682,7 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
     // V: 256 units of 4 keys x 8 dims, one per thread of the first 256
     __shared__ __attribute__((aligned(16))) _Float16 ks[2][kPfKeys][kHeadDim];
     __shared__ __attribute__((aligned(16))) _Float16 vt[2][kHeadDim][kPfVRow];
+    __shared__ int v_dropped;  // non-finite values were staged as zeros
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -694,7 +722,10 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
             vp[r] = load_b128(vr, v_unit ? off : kOOR);
         }
     };
-    auto stage = [&](int buf) {
+    const int wg_first = a.p0 + (int)blockIdx.x * TT * kPrefillTileTokens;  // a token's first position
+    if (tid == 0) v_dropped = 0;
+    auto stage = [&](int buf, int kb) {
+        if (kb * kPfKeys + kPfKeys - 1 > wg_first && drop_nonfinite(vp)) v_dropped = 1;
 #pragma unroll
         for (int r = 0; r < KP; ++r) {
             const int idx = tid + NT * r;
@@ -735,8 +766,8 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
                                     rope_freq(a.rope_base, d));
             rot_tab[row * kRotRow + d] = make_float2(rr.c, rr.s);
         }
-        __syncthreads();
     }
+    __syncthreads();
     const int rot_row = (wave / QPK) * kPrefillTileTokens + tl;
 
     // ---- this lane's query dims 32s + 8g + j (s = 0..3, j = 0..7): RMSNorm
@@ -794,7 +825,7 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
 #pragma unroll
     for (int d = 0; d < 8; ++d) o[d] = pf_float4{0.f, 0.f, 0.f, 0.f};
     const int blocks = last / kPfKeys + 1;
-    stage(0);
+    stage(0, 0);
     __syncthreads();
     for (int kb = 0; kb < blocks; ++kb) {
         const int buf = kb & 1;
@@ -896,8 +927,22 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
         }
         // the next block into the other buffer: every wave finished reading
         // it before the previous barrier
-        if (kb + 1 < blocks) stage(buf ^ 1);
+        if (kb + 1 < blocks) stage(buf ^ 1, kb + 1);
         __syncthreads();
+    }
+
+    // ---- non-finite values, to the tokens that attend them
+    if (__builtin_amdgcn_readfirstlane(v_dropped) != 0) {
+#pragma unroll 1
+        for (int key = (wg_first + 1) / kPfKeys * kPfKeys; key <= last; ++key) {
+            // (the largest offset added to kOOR stays past any cache too)
+            const uint32_t at = key <= pos ? ((uint32_t)key * kHeadDim + 4u * (uint32_t)g) * 2u : kOOR;
+#pragma unroll
+            for (int d = 0; d < 8; ++d) {
+                const float4 v = nonfinite_values(__builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(vr, (int)(at + 32u * d), 0, 0)));
+                o[d] += pf_float4{v.x, v.y, v.z, v.w};
+            }
+        }
     }
 
     // ---- the token's denominator over its four lanes, then O / l
@@ -988,6 +1033,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnAr
     constexpr int kLoop = 2 * KS * (int)sizeof(Buffer);
     __shared__ __attribute__((aligned(16))) char lds[kLoop > kPrologue ? kLoop : kPrologue];
     Buffer(*const bufs)[KS] = reinterpret_cast<Buffer(*)[KS]>(lds);
+    __shared__ int v_dropped;  // non-finite values were staged as zeros
 
     const int tid = threadIdx.x & (NT - 1);
     const int lane = tid & 63;
@@ -1037,8 +1083,11 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnAr
             vp[r] = load_b128(vr, v_unit ? off : kOOR);
         }
     };
-    auto stage_v = [&](int buf, const uint4 (&vp)[4]) {
+    const int wg_first = a.p0 + tile * TT * TOK;  // a token's first position
+    if (threadIdx.x == 0) v_dropped = 0;
+    auto stage_v = [&](int buf, int kb, uint4 (&vp)[4]) {
         if (v_unit) {
+            if (kb * kPfKeys + kPfKeys - 1 > wg_first && drop_nonfinite(vp)) v_dropped = 1;
             // row j of the unit: dim 8vc + j of keys 4va .. 4va + 3
             const uint32_t w[4][4] = {{vp[0].x, vp[0].y, vp[0].z, vp[0].w}, {vp[1].x, vp[1].y, vp[1].z, vp[1].w},
                                       {vp[2].x, vp[2].y, vp[2].z, vp[2].w}, {vp[3].x, vp[3].y, vp[3].z, vp[3].w}};
@@ -1165,7 +1214,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnAr
     // is wholly masked (its loads read zeros)
     const int rounds = (last / kPfKeys + KS) / KS;
     stage_k(0, kp0);
-    stage_v(0, vp0);
+    stage_v(0, half, vp0);
     __syncthreads();
     for (int round = 0; round < rounds; ++round) {
         const int kb = KS * round + half;
@@ -1284,7 +1333,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnAr
             }
         }
         __builtin_amdgcn_sched_group_barrier(kSchedMfma, 8, 0);
-        if (round + 1 < rounds) stage_v(buf ^ 1, vp);
+        if (round + 1 < rounds) stage_v(buf ^ 1, kb + KS, vp);
         __syncthreads();
     }
 
@@ -1311,6 +1360,23 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnAr
             const float w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int j = 0; j < 4; ++j) o[i >> 2][4 * (i & 3) + j] = o[i >> 2][4 * (i & 3) + j] * c0 + w[j] * c1;
+        }
+    }
+
+    // ---- non-finite values, to the tokens that attend them
+    if (__builtin_amdgcn_readfirstlane(v_dropped) != 0) {
+#pragma unroll 1
+        for (int key = (wg_first + 1) / kPfKeys * kPfKeys; key <= last; ++key) {
+            // (the largest offset added to kOOR stays past any cache too)
+            const uint32_t at = key <= pos ? ((uint32_t)key * kHeadDim + 4u * (uint32_t)h) * 2u : kOOR;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float4 v = nonfinite_values(__builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(vr, (int)(at + 16u * i), 0, 0)));
+                o[i >> 2][4 * (i & 3)] += v.x;
+                o[i >> 2][4 * (i & 3) + 1] += v.y;
+                o[i >> 2][4 * (i & 3) + 2] += v.z;
+                o[i >> 2][4 * (i & 3) + 3] += v.w;
+            }
         }
     }
 

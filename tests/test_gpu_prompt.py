@@ -415,3 +415,45 @@ def test_prompt_kv_pair(env, t, kvh, T):
     for got, ref in ((got_k, k), (got_v, v.reshape(T, kvh, 128))):
         assert max_rel_err(got.transpose(1, 0, 2), ref) <= 1e-3 + 2.0 ** -11
     dec.close()
+
+
+@pytest.mark.parametrize("qh,kvh,p0,T", [(8, 8, 0, 70), (16, 8, 5, 70), (32, 8, 61, 50), (64, 8, 0, 40),
+                                         (128, 128, 70, 129), (128, 64, 5, 139), (128, 32, 61, 192), (128, 16, 3, 487)])
+@pytest.mark.parametrize("what,value", [("v", np.inf), ("v", -7e4), ("v", np.nan), ("k", np.nan)])
+def test_chunk_attention_non_finite(env, qh, kvh, p0, T, what, value):
+    """A value (or key) that is not finite in the f16 cache reaches the tokens that attend it and no
+    other: in both forms of the chunk attention and every GQA width, tokens before it, other heads and
+    (for a value) other dims give the bits they give without it; -7e4 rounds to an f16 infinity."""
+    case(test="chunk_attention_non_finite", qh=qh, kvh=kvh, p0=p0, T=T, what=what, value=value)
+    E, per = env["E"], qh // kvh
+    cfg = dict(layers=1, hidden=4096, q_heads=qh, kv_heads=kvh, head_dim=128, ffn=256, vocab=1, rope_base=1.0e6,
+               epsilon=1.0e-6)
+    conf = E.AmdQwen3Config(**cfg)
+    cap = p0 + T
+    rng = np.random.default_rng(qh + kvh + p0 + T)
+    old = [rng.standard_normal((kvh, cap, 128)).astype(np.float16) for _ in range(2)]
+    q = rng.standard_normal((T, qh * 128)).astype(np.float32)
+    kv = {nm: rng.standard_normal((T, kvh * 128)).astype(np.float32) for nm in "kv"}
+    qn, kn = to_dev(synth.gamma_numpy(128, 1)), to_dev(synth.gamma_numpy(128, 2))
+
+    def run(k, v):
+        cache = E.AmdKvCache(env["ctx"], conf, cap)
+        for ptr, dev in zip(cache.layer(0), old):
+            assert env["ctx"]._lib.ribn_amd_memcpy_htod(env["ctx"].handle, ctypes.c_void_p(ptr),
+                                                        dev.ctypes.data_as(ctypes.c_void_p), dev.nbytes) == 0
+        out = to_dev(np.zeros(T * qh * 128, np.float32))
+        E.attention_prefill(env["ctx"], conf, cache, 0, to_dev(q.reshape(-1)), to_dev(k.reshape(-1)), to_dev(v.reshape(-1)),
+                            qn, kn, T, p0, out)
+        return to_host(out, env["ctx"]).reshape(T, kvh, per, 128)
+
+    want = run(kv["k"], kv["v"])
+    assert np.all(np.isfinite(want))
+    for at in (T // 2 + 3, T - 2):
+        head, dim = at % kvh, (37 * at) % 128
+        bad = {nm: a.copy() for nm, a in kv.items()}
+        bad[what][at, head * 128 + dim] = value
+        got = run(bad["k"], bad["v"])
+        reached = got[at:, head, :, dim] if what == "v" else got[at:, head]
+        assert not np.any(np.isfinite(reached)), at
+        reached[...] = (want[at:, head, :, dim] if what == "v" else want[at:, head])
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), at

@@ -1456,22 +1456,25 @@ hipError_t launch_kv_append(const AttnArgs& args, int members, hipStream_t strea
 }
 
 namespace {
-// Whether the wide form's grid fills enough of the 256 CUs (its workgroups take
-// one each, with a longer prologue). Measured, us, narrow / wide: 32 / 8 heads at
-// 512, 768, 1,024, 2,047 tokens (128, 192, 256, 512 workgroups) 27.0 / 29.2,
-// 41.5 / 37.2, 53.5 / 45.6, 139 / 96; 16 / 8 heads at 1,024, 1,400 (128, 176)
-// 40.6 / 42.0, 57.5 / 53.6; 8 / 8 heads at 1,024 (64) 45.4 / 41.0; 64 / 8 heads at
-// 512, 1,024 (128, 256) 31.0 / 42.9, 81.5 / 70.1.
-bool wide_prefill(const PrefillAttnArgs& a, int tiles) {
+// Whether the wide form's grid fills enough of the CUs (its workgroups take one
+// each, with a longer prologue): 11/16 of them, a quarter with one query head per KV
+// head, all with eight. Measured on 256 CUs, narrow time / wide time by workgroups,
+// whole calls from position 0: two heads (16 / 8) 128 1.00, 136 1.09, 160 1.17, 168 1.20,
+// 176 1.15; four (32 / 8) 128 0.91, 144 1.07, 168 1.11, 176 1.04, 192 1.14, but (64 / 16
+// heads, shorter chunks) 128 0.88, 160 0.95, 176 0.99, 192 1.01; one (8 / 8, 16 / 16, 4 / 4)
+// 32 1.11, 48 1.10, 64 1.08-1.16, so the line could lie lower; eight (64 / 8) 176 0.98, 200
+// 1.02, 240 1.09, 256 1.15, (32 / 4) 128 0.69, 152 0.84, 188 1.03, 228 1.07. After 1,000
+// cached tokens the wide form gains more everywhere.
+bool wide_prefill(const PrefillAttnArgs& a, int tiles, int cu_count) {
     const int qpk = a.q_heads / a.kv_heads;
-    return tiles * a.kv_heads >= (qpk == 1 ? 64 : qpk == 8 ? 256 : 176);
+    return 16 * tiles * a.kv_heads >= (qpk == 1 ? 4 : qpk == 8 ? 16 : 11) * cu_count;
 }
 
 template <int QPK>
-hipError_t launch_prefill_heads(const PrefillAttnArgs& a, hipStream_t stream) {
+hipError_t launch_prefill_heads(const PrefillAttnArgs& a, int cu_count, hipStream_t stream) {
     constexpr int TT = QPK < 4 ? 4 / QPK : 1;  // token tiles per workgroup
     const int wide = (a.tokens + kPrefillWideTokens * TT - 1) / (kPrefillWideTokens * TT);
-    if (wide_prefill(a, wide)) {
+    if (wide_prefill(a, wide, cu_count)) {
         hipLaunchKernelGGL(attn_prefill_wide_kernel<QPK>, dim3((unsigned)wide * (unsigned)a.kv_heads), dim3(512), 0, stream, a, wide);
     } else {
         const int tiles = (a.tokens + kPrefillTileTokens * TT - 1) / (kPrefillTileTokens * TT);
@@ -1481,7 +1484,7 @@ hipError_t launch_prefill_heads(const PrefillAttnArgs& a, hipStream_t stream) {
 }
 }  // namespace
 
-hipError_t launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream) {
+hipError_t launch_prefill_attention(const PrefillAttnArgs& a, int cu_count, hipStream_t stream) {
     if (a.tokens < 1 || a.kv_heads < 1 || a.q_heads % a.kv_heads != 0 || a.p0 < 0 ||
         (long long)a.p0 + a.tokens > a.mem.capacity || a.mem.keys == nullptr || a.mem.values == nullptr) {
         return hipErrorInvalidValue;
@@ -1490,10 +1493,10 @@ hipError_t launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t stream
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.out == nullptr) return e;
     switch (a.q_heads / a.kv_heads) {
-    case 1: return launch_prefill_heads<1>(a, stream);
-    case 2: return launch_prefill_heads<2>(a, stream);
-    case 4: return launch_prefill_heads<4>(a, stream);
-    case 8: return launch_prefill_heads<8>(a, stream);
+    case 1: return launch_prefill_heads<1>(a, cu_count, stream);
+    case 2: return launch_prefill_heads<2>(a, cu_count, stream);
+    case 4: return launch_prefill_heads<4>(a, cu_count, stream);
+    case 8: return launch_prefill_heads<8>(a, cu_count, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -130,7 +130,7 @@ constexpr int kPrefillWideTokens = 32;
 // The chunk's K (RMSNorm + rope) and V stored as f16 at their positions, then
 // (when `out` is set) causal attention of every token over positions
 // 0 .. its own on the matrix cores. q_heads / kv_heads in {1, 2, 4, 8}.
-hipError_t launch_prefill_attention(const PrefillAttnArgs& args, hipStream_t stream);
+hipError_t launch_prefill_attention(const PrefillAttnArgs& args, int cu_count, hipStream_t stream);
 
 // Slice results a two-stage greedy selection keeps per member.
 constexpr int kArgmaxSlices = 64;

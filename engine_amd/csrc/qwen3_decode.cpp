@@ -608,7 +608,7 @@ hipError_t enqueue_prompt_chunk(ribn_amd_qwen3_decode* d, ribn_amd_kv_cache* cac
         a.eps = c.epsilon;
         a.rope_base = c.rope_base;
         a.scale = 1.4426950408889634f / sqrtf((float)c.head_dim);
-        e = ribn_amd::launch_prefill_attention(a, stream);
+        e = ribn_amd::launch_prefill_attention(a, d->ctx->cu_count, stream);
         if (e != hipSuccess || last) break;
         e = ribn_amd::launch_act_f16(false, d->p_attn, nullptr, 0.f, tokens, qdim, d->p_gemm, stream);
         if (e == hipSuccess) e = prompt_gemm(d, L.attn_output, d->p_y, tokens, stream);
@@ -815,7 +815,7 @@ ribn_amd_status ribn_amd_attention_prefill(ribn_amd_context* ctx, const ribn_amd
     a.eps = config->epsilon;
     a.rope_base = config->rope_base;
     a.scale = 1.4426950408889634f / sqrtf((float)config->head_dim);
-    hipError_t e = ribn_amd::launch_prefill_attention(a, ctx->stream);
+    hipError_t e = ribn_amd::launch_prefill_attention(a, ctx->cu_count, ctx->stream);
     return e == hipSuccess ? ok() : driver(e, "prompt attention launch");
 }
 

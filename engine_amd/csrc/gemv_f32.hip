@@ -33,6 +33,7 @@
 //   T   = ((P_0 + P_1) + P_2) ... in slice order,
 //   y   = T * inv with inv = 1/sqrt(sum(x^2)/K + eps) for RMSNorm (else y = T),
 //   sum(x^2) = per 256-element block, a fixed lane tree; blocks added in order.
+#include "per_device.hpp"
 #include "wave_rows.hpp"
 
 #include <algorithm>
@@ -1503,10 +1504,13 @@ struct F32Instance {
     static hipError_t launch(const WaveGemvArgs& a, int cu_count, int per_cu, hipStream_t stream) {
         auto kern = gemv_f32_kernel<T, MT, PRO, ONE_SLICE, NBUF, WAVES, GROUP, PAIR, SPLIT>;
         const size_t lds = f32_lds_bytes<T>(MT, ONE_SLICE ? std::min(a.K, (int)kSliceElems) : a.K);
+        const int max_lds = (int)f32_lds_bytes<T>(MT, ONE_SLICE ? kSliceElems : kWaveMaxK);
+        static PerDevice sized;
+        (void)sized.once(a.device, [&] {
+            return hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+        });
         int occ = occupancy.load(std::memory_order_relaxed);
         if (occ == 0) {
-            const int max_lds = (int)f32_lds_bytes<T>(MT, ONE_SLICE ? kSliceElems : kWaveMaxK);
-            (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)kern, WAVES * 64, max_lds) !=
                     hipSuccess ||
                 occ < 1) {
@@ -1584,12 +1588,11 @@ hipError_t launch_slices(const WaveGemvArgs& a, int cu_count, hipStream_t stream
     constexpr int kRing = 2;
     constexpr int kMaxLds = 158 * 1024;  // beside the kernel's own few hundred bytes
     auto kern = gemv_f32_slices_kernel<T, MT, PRO, MULTI, kRing, PAIR>;
-    static std::atomic<bool> sized{false};
-    if (!sized.load(std::memory_order_relaxed)) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
-        if (e != hipSuccess) return e;
-        sized.store(true, std::memory_order_relaxed);
-    }
+    static PerDevice sized;
+    const hipError_t e = sized.once(a.device, [&] {
+        return hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+    });
+    if (e != hipSuccess) return e;
     const int nb = a.K >> 8, slices = (nb + 15) >> 4;
     long long quads = 0;
     for (int i = 0; i < (PAIR ? 1 : a.count); ++i)
@@ -1683,13 +1686,11 @@ template <int T, int MG, int PRO, bool PAIR, bool SPLIT = false>
 hipError_t launch_many_instance(const WaveGemvArgs& a, int cu_count, hipStream_t stream) {
     constexpr int kRing = 2;
     auto kern = gemv_f32_many_kernel<T, MG, PRO, kRing, PAIR, SPLIT>;
-    static std::atomic<bool> sized{false};
-    if (!sized.load(std::memory_order_relaxed)) {
-        const hipError_t e =
-            hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, MG * kManyLds);
-        if (e != hipSuccess) return e;
-        sized.store(true, std::memory_order_relaxed);
-    }
+    static PerDevice sized;
+    const hipError_t e = sized.once(a.device, [&] {
+        return hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, MG * kManyLds);
+    });
+    if (e != hipSuccess) return e;
     const int nb = a.K >> 8;
     const int slices = SPLIT ? (nb + 15) >> 4 : 1;
     long long units = 0;

@@ -34,6 +34,7 @@
 // batched launch is bit-identical to the single-member launch.
 #include "kquant_device.hpp"
 #include "kquant_launch.hpp"
+#include "per_device.hpp"
 #include "wave_rows.hpp"
 
 #include <algorithm>
@@ -627,10 +628,13 @@ struct WaveInstance {
     static hipError_t launch(const WaveGemvArgs& a, int cu_count, int per_cu, hipStream_t stream) {
         auto kern = gemv_wave_kernel<T, MT, PRO, ONE_SLICE, NBUF, WAVES, GROUP, PAIR>;
         const size_t lds = act_lds_bytes<T>(MT, a.K);
+        const int max_lds = (int)act_lds_bytes<T>(MT, ONE_SLICE ? kSliceElems : kWaveMaxK);
+        static PerDevice sized;
+        (void)sized.once(a.device, [&] {
+            return hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+        });
         int occ = occupancy.load(std::memory_order_relaxed);
         if (occ == 0) {
-            const int max_lds = (int)act_lds_bytes<T>(MT, ONE_SLICE ? kSliceElems : kWaveMaxK);
-            (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)kern, WAVES * 64, max_lds) !=
                     hipSuccess ||
                 occ < 1) {

@@ -76,6 +76,7 @@ struct WaveGemvArgs {
     // input x equal to fold->y) adds pending sums into x first.
     F32MmaFold* defer;
     const F32MmaFold* fold;
+    int device;  // the launch's device
 };
 
 constexpr int kArithF32 = 0;

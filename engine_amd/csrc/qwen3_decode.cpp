@@ -206,6 +206,7 @@ hipError_t wave(const ribn_amd_qwen3_decode* d, const ribn_amd_quantized_weight*
     for (int m0 = 0; m0 < members; m0 += per) {
         const int mc = std::min(per, members - m0);
         ribn_amd::WaveGemvArgs a{};
+        a.device = d->ctx->device;
         int rows = 0;
         for (int i = 0; i < count; ++i) {
             const int n = (int)ws[i]->output_size;

@@ -192,6 +192,7 @@ ribn_amd_status launch_wave_group(ribn_amd_gemv* g, const ribn_amd_quantized_wei
     for (size_t m0 = 0; m0 < members; m0 += (size_t)per_launch) {
         const size_t mc = std::min<size_t>((size_t)per_launch, members - m0);
         ribn_amd::WaveGemvArgs a{};
+        a.device = g->ctx->device;
         int rows = 0;
         for (size_t i = 0; i < count; ++i) {
             const uint64_t n = ws[i]->output_size;
@@ -937,6 +938,7 @@ ribn_amd_status ribn_amd_gemv_execute_gate_up_swiglu(ribn_amd_gemv* g, const rib
     for (size_t m0 = 0; m0 < members; m0 += (size_t)per_launch) {
         const size_t mc = std::min<size_t>((size_t)per_launch, members - m0);
         ribn_amd::WaveGemvArgs a{};
+        a.device = g->ctx->device;
         a.w[0] = gate->data;
         a.wbytes[0] = (uint32_t)gate->encoded_bytes;
         a.w[1] = up->data;

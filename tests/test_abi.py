@@ -3,6 +3,7 @@ header declares, and its host-only validation mirrors the reference's
 validate_quantized_geometry (crates/nvidia/src/quantized.rs:1755-1804).
 No kernel is launched here."""
 import ctypes
+import os
 import subprocess
 
 import pytest
@@ -121,3 +122,13 @@ def test_decoder_keeps_its_weights_and_norms_alive():
     del dec
     gc.collect()
     assert all(r() is None for r in refs)
+
+
+def test_per_device_setup(tmp_path):
+    """A kernel's one-time set-up (its LDS attribute) runs on every device it is launched on."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    exe = tmp_path / "per_device_test"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-pthread", "-I",
+                    os.path.join(os.path.dirname(here), "engine_amd", "csrc"), os.path.join(here, "cpp", "per_device_test.cpp"),
+                    "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.strip() == "ok"

@@ -74,6 +74,7 @@
 // shape: its bits do not change with the other members' values, their count
 // (from 9 members on) or its position in the batch.
 #include "kquant_device.hpp"
+#include "f32mma_shape.hpp"
 #include "kquant_launch.hpp"
 
 #include <float.h>
@@ -947,50 +948,6 @@ template <int T, int R, int MT> constexpr int ring_depth() {
     constexpr int nl = lds_slots<T, MT>();
     return nl == 2 ? (R == 1 ? 4 : 2) : nl;
 }
-// Launch shape of one product: compute waves per workgroup, the K split and
-// the row groups. The split comes from the weight shape alone (row tiles,
-// super-blocks and the partial room a 64-member launch needs), never from the
-// member count, so a member's sums are added in the same order whatever the
-// batch: among the one-tile-per-wave shapes whose grid fits the CUs in one
-// round (all workgroups resident at once), the one with the fewest (row tile
-// x super-block) units per workgroup sets it (ties: more compute waves, which
-// share the LDS fragments, then fewer splits). Measured on MI355X at the
-// Qwen3-8B FFN shapes, two row tiles per wave (halving the LDS fragment
-// reads) ran M = 64 slower: 96.0 against 80.3 us per FFN.
-struct F32MmaShape {
-    int waves, splits, split_blocks, groups;
-};
-constexpr int kF32MmaMaxComputeWaves = 7;  // plus the loader: eight waves, two per SIMD
-F32MmaShape f32mma_split(int tiles, int nb, int max_splits, int cu_count) {
-    constexpr int kMaxWaves = kF32MmaMaxComputeWaves;
-    F32MmaShape best{kMaxWaves, 1, nb, (tiles + kMaxWaves - 1) / kMaxWaves};
-    long best_cost = -1;
-    for (int s = 1; s <= std::min(nb, std::max(1, max_splits)); ++s) {
-        const int sbk = (nb + s - 1) / s;
-        if ((nb + sbk - 1) / sbk != s) continue;  // the same split as a smaller s
-        for (int w = 1; w <= kMaxWaves; ++w) {
-            const int groups = (tiles + w - 1) / w;
-            if ((long)groups * s > cu_count) continue;
-            const long cost = (long)w * sbk;
-            const bool better = best_cost < 0 || cost < best_cost ||
-                                (cost == best_cost && (w > best.waves || (w == best.waves && s < best.splits)));
-            if (better) {
-                best = {w, s, sbk, groups};
-                best_cost = cost;
-            }
-        }
-    }
-    return best;
-}
-// The same split with R row tiles per wave (gate/up pairs: 2): the fewest
-// compute waves that still fit the grid in one round.
-F32MmaShape f32mma_shape_r(const F32MmaShape& one, int tiles, int R, int cu_count) {
-    const int units = (tiles + R - 1) / R;
-    const int max_groups = std::max(1, cu_count / one.splits);
-    const int w = std::min(kF32MmaMaxComputeWaves, std::max(1, (units + max_groups - 1) / max_groups));
-    return {w, one.splits, one.split_blocks, (units + w - 1) / w};
-}
-
 // The one-wave kernels, instantiated here so that they lie together in the code
 // object, before the two-wave ones that launch_shape would put between them. A
 // layer's kernels (56 KB of code at 16 members) about fill the instruction cache
@@ -1019,13 +976,7 @@ hipError_t launch_shape(F32MmaArgs a, const F32MmaShape& sh, hipStream_t stream)
     const dim3 grid((unsigned)sh.groups, (unsigned)sh.splits);
     bool launched = false;
     if constexpr (PAIR && MT % 2 == 0) {
-        // Where a workgroup holds one unit, and for Q4_K at four member tiles.
-        // Measured, gate/up at 24 / 64 members, us, one wave a unit / two:
-        // 4096 -> 2 x 4096 (one unit) Q4_K 21.9 / 20.7 and 31.0 / 26.9, Q6_K
-        // 42.9 / 40.4 and 82.5 / 77.7; 4096 -> 2 x 12288 (three) Q4_K 32.7 / 37.0
-        // and 48.4 / 46.7, Q5_K 38.2 / 45.4 and 54.2 / 55.7. (Single products
-        // were slower with two at every shape tried.)
-        if (sh.waves == 1 || (T == kQ4K && MT == 4 && 2 * sh.waves + 1 <= 8)) {
+        if (f32mma_two_waves(T == kQ4K, MT, sh)) {
             hipLaunchKernelGGL((f32mma_gemv_kernel<T, R, MT, PAIR, lds_slots<T, MT>(), ring_depth<T, R, MT>(), 2>), grid,
                                dim3(64 * (2 * sh.waves + 1)), 0, stream, a);
             launched = true;
@@ -1056,8 +1007,7 @@ hipError_t launch_t(const F32MmaArgs& a, size_t partial_bytes, int cu_count, F32
     const bool pair = a.pair_swiglu != 0;
     const int tiles = pair ? 2 * ((a.rows_end[0] + 15) / 16) : (a.total_rows + 15) / 16;
     const int vrows = pair ? 2 * a.rows_end[0] : a.total_rows;
-    const size_t split_bytes = (size_t)kStep * (size_t)vrows * 4;
-    const int max_splits = a.partial == nullptr ? 1 : (int)std::min<size_t>(16, partial_bytes / split_bytes);
+    const int max_splits = a.partial == nullptr ? 1 : f32mma_max_splits(kStep, vrows, partial_bytes);
     const F32MmaShape one = f32mma_split(tiles, nb, max_splits, cu_count);
     // an accumulating single-weight product of one launch may leave its split
     // sums to the next call (F32MmaFold)

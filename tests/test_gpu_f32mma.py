@@ -233,11 +233,22 @@ def test_config2_ffn_shapes(env, members):
             assert max_rel_err(got[nm][m], O.quant_gemv(t, e, k, n, src[m], threads=16)) <= F32_RTOL, (nm, m)
 
 
-@pytest.mark.parametrize("t,k,n,members", [(12, 512, 48, 24), (13, 768, 272, 64), (14, 512, 304, 33), (12, 1024, 4096, 50),
-                                           (12, 512, 12304, 61)])
+# Gate/up pairs (type, K, N, members) and their shape on 256 CUs: units a workgroup, K splits, waves a
+# unit. The shapes are checked on the host by tests/test_f32mma_shape.py, so a changed rule cannot
+# move a case off its path unseen.
+PAIR_SHAPES = {
+    (12, 512, 48, 24): (1, 2, 2), (13, 768, 272, 64): (1, 3, 2), (14, 512, 304, 33): (1, 2, 2),
+    (12, 1024, 4096, 50): (2, 2, 2),
+    # seven waves a workgroup, whole and ragged last tiles and workgroups
+    (12, 4096, 12288, 61): (3, 1, 2), (12, 512, 12279, 64): (3, 1, 2), (12, 256, 8200, 49): (3, 1, 2),
+    # the first shapes past the two-wave form, and other types at three units
+    (12, 512, 12304, 61): (4, 1, 1), (13, 512, 12280, 61): (3, 1, 1), (14, 512, 12280, 33): (3, 1, 1)}
+
+
+@pytest.mark.parametrize("t,k,n,members", list(PAIR_SHAPES))
 def test_gate_up_pair_two_waves_a_unit(env, t, k, n, members):
-    """Gate/up pairs whose member tiles two waves share (one unit a workgroup; Q4_K at four tiles):
-    silu(gate) * up of the separate products (the same chains per member, summed alike up to their
+    """Gate/up pairs whose member tiles two waves share (one unit a workgroup; Q4_K at four tiles), and
+    the first ones past that: silu(gate) * up of the separate products (the same chains per member, summed alike up to their
     split), and members bit-identical to a 9-member call."""
     case(test="pair_two_waves", t=t, k=k, n=n, members=members)
     ws = [upload(env, t, k, n, synth.kquant_numpy(t, k, n, seed=k + n + j)) for j in range(2)]

@@ -825,7 +825,7 @@ def check_dispatch_line(env, t, blocks, at, members, pro):
 
 
 @pytest.mark.parametrize("t,blocks,at", [(12, 112, 512), (13, 68, 512), (14, 68, 3072), (14, 66, 4096), (12, 80, 4096),
-                                         (13, 100, 2048)])
+                                         (13, 100, 2048), (14, 128, 512)])
 def test_long_k_dispatch_lines(env, t, blocks, at):
     """As above for one member of K beyond 16384, between one launch and the slice split."""
     check_dispatch_line(env, t, blocks, at, 1, "")

@@ -753,8 +753,8 @@ namespace {
 // Measured, one member, us (before: one row a unit, or pairs of rows over all
 // slices): Q4_K 5120 -> 17408 23.6 -> 16.3, Q6_K 29.7 -> 22.0; Q4_K 12288 ->
 // 17408 38.0 -> 32.0; 1024 -> 17408 8.9 -> 6.3; two members 5120 -> 17408 30.4 ->
-// 20.9. What bounds it: 3.1-4.0 TB/s of weights after a 4-6 us ramp; the
-// choice of form is launch_few's.
+// 20.9. What bounds it: 3.1-4.0 TB/s of weights after a 4-6 us ramp. Where it
+// serves is chosen by launch_few (pairs_form) and launch_split (one_launch_long_k).
 constexpr int kSliceWaves = 8;
 
 // Rows of one slice a unit takes.
@@ -1080,7 +1080,9 @@ __global__ __launch_bounds__(kSliceWaves * 64) void gemv_f32_slices_kernel(WaveG
 // 4 x 4 outer products, D[i][j] += x_i * q_j, each element one fused f32
 // multiply-add (checked bit for bit against fmaf over normal, denormal,
 // overflowing, infinite and NaN operands), so a chain of them over a scale
-// group's elements is the S_g of the single-member kernel, in its order.
+// group's elements is the S_g of the single-member kernel, in its order. (The
+// minimum terms m * X are formed onto +0, so one of -0 becomes +0: a row of zero
+// weights may give the other zero.)
 //
 // Mapping. A wave owns one quarter of the slice (4 super-blocks, 16 lane
 // records) and walks units of 4 rows x that quarter: lane l holds record

@@ -245,11 +245,11 @@ ribn_amd_status ribn_amd_gemv_execute(ribn_amd_gemv *gemv, const ribn_amd_quanti
 /* execute_warp (quantized.rs:401-435): the wave64 bandwidth kernel (default
  * decode path), in the kernel object's GEMV mode. K up to 16384 stages in one
  * launch; a K of 16640..65536 (e.g. the 17408-wide down projection of the
- * reference's 27B shapes) runs the f32 arithmetic in either mode: one launch
- * for one member up to 32768, else the slice-split form (one 4096-wide slice
- * per workgroup, slice totals added in order by a second launch; plain,
- * grouped and accumulating products); a larger K runs the exact-order
- * kernel. */
+ * reference's 27B shapes) runs the f32 arithmetic in either mode: the
+ * slice-split form (one 4096-wide slice per workgroup, slice totals added in
+ * order by a second launch), or one launch with the same bits for one member up
+ * to 32768 where that is faster (plain, grouped and accumulating products); a
+ * larger K runs the exact-order kernel. */
 ribn_amd_status ribn_amd_gemv_execute_warp(ribn_amd_gemv *gemv, const ribn_amd_quantized_weight *weight,
                                            const float *input, size_t input_len, float *output,
                                            size_t output_len);

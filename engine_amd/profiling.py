@@ -156,7 +156,7 @@ def decode_steps_summary(path: str, steps: int = 32) -> list[dict]:
 
 
 # Kernels only the prompt prefill launches (ribn_amd_qwen3_prefill_prompt).
-PROMPT_KERNELS = ("act_f16_kernel", "qgemm", "attn_prefill_kernel", "kv_append_seq_kernel")
+PROMPT_KERNELS = ("act_f16_kernel", "qgemm", "attn_prefill_", "kv_append_seq_kernel")
 
 
 def prompt_summary(path: str, prompts: int = 1) -> dict:

@@ -123,3 +123,12 @@ def test_prompt_summary_keeps_prompt_kernels_only(tmp_path):
     assert names == ["qgemm_tile_kernel<12, 3, 8>", "attn_prefill_kernel<4>", "act_f16_kernel<false, true, 0>"]
     assert w["kernels"][0][2:] == (1.0, 10.0, 10.0)
     assert abs(w["busy_us"] - 15.0) < 1e-9
+
+
+def test_prompt_summary_knows_the_prompt_kernels(tmp_path):
+    """Every kernel of the prompt path alone is in the summary, the many-token attention too."""
+    names = ("act_f16_kernel<false, true, 0>", "qgemm_reduce_kernel<4>", "qgemm_tile_kernel<12, 4, 8>", "kv_append_seq_kernel",
+             "attn_prefill_kernel<4>", "attn_prefill_wide_kernel<4>")
+    _write_trace(tmp_path / "run_kernel_trace.csv",
+                 [(f"void ribn_amd::{n}(int)", (64, 1, 1), 10000 * i, 10000 * i + 1000) for i, n in enumerate(names + ("attn_decode_kernel<4>",))])
+    assert sorted(k[0] for k in P.prompt_summary(str(tmp_path))["kernels"]) == sorted(names)

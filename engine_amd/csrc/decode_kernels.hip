@@ -659,7 +659,7 @@ __device__ __forceinline__ bool drop_nonfinite(uint4 (&vp)[4]) {
     uint32_t bad = 0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) bad |= nonfinite_halfs(vp[r].x) | nonfinite_halfs(vp[r].y) | nonfinite_halfs(vp[r].z) | nonfinite_halfs(vp[r].w);
-    if (bad == 0) return false;
+    if (__builtin_expect(bad == 0, 1)) return false;
     auto finite = [](uint32_t w) { return w & ~((nonfinite_halfs(w) >> 15) * 0xffffu); };
 #pragma unroll
     for (int r = 0; r < 4; ++r) vp[r] = make_uint4(finite(vp[r].x), finite(vp[r].y), finite(vp[r].z), finite(vp[r].w));
@@ -932,7 +932,7 @@ __global__ __launch_bounds__(64 * (QPK < 4 ? 4 : QPK)) void attn_prefill_kernel(
     }
 
     // ---- non-finite values, to the tokens that attend them
-    if (__builtin_amdgcn_readfirstlane(v_dropped) != 0) {
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(v_dropped) != 0, 0)) {
 #pragma unroll 1
         for (int key = (wg_first + 1) / kPfKeys * kPfKeys; key <= last; ++key) {
             // (the largest offset added to kOOR stays past any cache too)
@@ -1364,7 +1364,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_wide_kernel(PrefillAttnAr
     }
 
     // ---- non-finite values, to the tokens that attend them
-    if (__builtin_amdgcn_readfirstlane(v_dropped) != 0) {
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(v_dropped) != 0, 0)) {
 #pragma unroll 1
         for (int key = (wg_first + 1) / kPfKeys * kPfKeys; key <= last; ++key) {
             // (the largest offset added to kOOR stays past any cache too)
